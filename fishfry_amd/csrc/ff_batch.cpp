@@ -226,6 +226,7 @@ bool col_desc(const PassLaunch& r, MultiColDesc& out, size_t& lds) {
   const ColArgs& c = r.col;
   if (r.blue || r.groups != 1 || r.split || c.outer_fast) return false;
   if (c.in.nlo || c.xtw || c.imap_n2 || c.jmap_n1) return false;  // four-step lines
+  if (c.mix) return false;                                        // mixed-radix lines
   if (c.in.nb != 1 || c.out.nb != 1 || c.in.lgKT < 30 || c.out.lgKT < 30 || c.nline != c.lp.n) return false;
   if (!multi_kernel_exists(MULTI_COL, r.f32, r.sel, 0)) return false;
   const int v = multi_col_variant(c.lp.n, r.E, c.lp);
@@ -260,7 +261,7 @@ bool col_desc(const PassLaunch& r, MultiColDesc& out, size_t& lds) {
 
 bool row_desc(const PassLaunch& r, MultiRowDesc& out, size_t& lds) {
   const RowArgs& c = r.row;
-  if (r.blue || r.odd || c.nline != c.lp.n) return false;
+  if (r.blue || r.odd || c.mix || c.nline != c.lp.n) return false;
   if (r.kind == 2 && c.spec.lgKT < 30) return false;  // z inverse of a blocked spectrum
   const int kind = r.kind == 1 ? MULTI_R2C : MULTI_C2R;
   if (!multi_kernel_exists(kind, r.f32, r.sel, r.kind == 2 ? r.epi : 0)) return false;
@@ -674,6 +675,9 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
       for (auto& kv : keys) {
         // four-step lines have no single configuration to tune
         if ((kv[0] == 1 && p->fy.n) || (kv[0] == 2 && p->fx.n) || ((kv[0] == 0 || kv[0] == 3) && p->fz.n)) continue;
+        // nor have mixed-radix ones
+        const MixCfg* mix[4] = {&p->mzr[prec], &p->my[prec], &p->mx[prec], &p->mzi[prec]};
+        if (mix[kv[0]]->plan) continue;
         if (!seen.count({kv[0], kv[1], prec})) seen[{kv[0], kv[1], prec}] = i;
       }
     }

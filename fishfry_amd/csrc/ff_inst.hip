@@ -4,6 +4,7 @@
 #include <type_traits>
 
 #include "ff_kernels.hpp"
+#include "ff_mixed.hpp"
 
 #ifndef FF_E
 #error "FF_E must be defined"
@@ -101,10 +102,13 @@ static const void* col_static_fn(int f32, int split, int mode, int n, int T, int
 }
 
 // Bluestein lines use the default kernel shape (one group, complex exchange).
+// Mixed-radix passes (a.mix) have no elements per thread: they dispatch as E = 1.
 template <>
 hipError_t PassLaunchers<FF_E>::col(int f32, int mode, int split, int groups, int blue, int stat, const Launch& l,
                                     const ColArgs& a) {
   const void* fn = nullptr;
+  if constexpr (FF_E == 1)
+    if (a.mix) return mix_col(f32, mode, l, a);
   if (stat) {
     fn = col_static_fn<0>(f32, split, mode, a.lp.n, a.T, stat);
   } else if (blue) {
@@ -156,6 +160,8 @@ static const void* r2c_static_fn(int f32, int in_f32, int odd, int M, int stat) 
 template <>
 hipError_t PassLaunchers<FF_E>::r2c(int f32, int in_f32, int odd, int blue, int stat, const Launch& l,
                                     const RowArgs& a) {
+  if constexpr (FF_E == 1)
+    if (a.mix) return mix_r2c(f32, in_f32, odd, l, a);
   const void* fn = stat ? r2c_static_fn<0>(f32, in_f32, odd, a.lp.n, stat)
                         : (blue ? r2c_fn<true>(f32, in_f32, odd) : r2c_fn<false>(f32, in_f32, odd));
   if (!fn) return hipErrorInvalidValue;
@@ -205,6 +211,8 @@ static const void* c2r_static_fn(int f32, int out_kind, int odd, int epi, int M,
 template <>
 hipError_t PassLaunchers<FF_E>::c2r(int f32, int out_kind, int odd, int epi, int blue, int stat, const Launch& l,
                                     const RowArgs& a) {
+  if constexpr (FF_E == 1)
+    if (a.mix) return mix_c2r(f32, out_kind, odd, epi, l, a);
   const void* fn = stat ? c2r_static_fn<0>(f32, out_kind, odd, epi, a.lp.n, stat)
                         : (blue ? c2r_fn<true>(f32, out_kind, odd, epi) : c2r_fn<false>(f32, out_kind, odd, epi));
   if (!fn) return hipErrorInvalidValue;

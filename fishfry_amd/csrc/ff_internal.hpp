@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -64,6 +65,9 @@ void push_bluestein(std::vector<unsigned char>& buf, int n, int m, int prec, siz
 const void* table_twiddle(int n, int prec);
 const void* table_post(int nz, int prec);
 bool table_bluestein(int n, int m, int prec, const void* out[3]);
+// A table of the caller's making, under a kind of its own (above 3).
+using TableBuilder = std::function<void(std::vector<unsigned char>&)>;
+const void* table_built(int kind, int n, int prec, const TableBuilder& build);
 // Finite-difference factor table g[k] = 4 sin^2(pi k/n) (order 3) or
 // 4 sin^2(pi k/n) (1 + sin^2(pi k/n)/3) (order 5), k < n, FP64.
 const double* table_symbol(int n, int order);

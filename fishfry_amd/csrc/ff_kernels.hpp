@@ -130,6 +130,8 @@ struct ColArgs {
   int nline;                     // transform length (lp.n: engine length; larger for Bluestein)
   const void *chirp, *bsf, *bsi;  // Bluestein tables (see line_dft)
   const PassInst* inst;           // grouped launch: per-instance fields (null: one solve)
+  const void* mix;                // the MixPlan of a mixed-radix pass, in device memory (null: none)
+  int nbuf;                       // its LDS buffers
 };
 
 // Buffers in global memory.  The per-instance fields come either from the
@@ -575,6 +577,10 @@ struct RowArgs {
   int nline;                     // transform length M (lp.n: engine length; larger for Bluestein)
   const void *chirp, *bsf, *bsi;  // Bluestein tables (see line_dft)
   const PassInst* inst;           // grouped launch: per-instance fields (null: one solve)
+  const void* mix;                // the MixPlan of a mixed-radix pass, in device memory (null: none)
+  long long nlines;               // mixed-radix pass: lines (rows, or for odd nz pairs of them);
+  int lgT;                        // T = 2^lgT; Linv = ceil(2^32 / half-spectrum steps per line) and
+  uint32_t hyinv;                 // ceil(2^32 / pairs per plane)
   int m1;                         // four-step z rows: the stride-1 sub-line length (ff_zsplit.hip)
   int lone;                       // odd nz, nx*ny odd: the launch's one pair is the last row alone
                                   // (no second row: zero on the way in, not written on the way out)

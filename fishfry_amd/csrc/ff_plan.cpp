@@ -177,8 +177,9 @@ struct TableEntry {
 // Builds a table on the host, uploads it once per device and keeps it until
 // the process ends; kind 0: W_n[t], t < n; 1: exp(-2 pi i k/n), k < n/2 (at
 // least one entry); 2: the Bluestein tables of length n over m; 3: the
-// finite-difference factors of order m, k < n (FP64).
-static const TableEntry* table_entry(int kind, int n, int m, int prec) {
+// finite-difference factors of order m, k < n (FP64); others: what build
+// writes (table_built).
+static const TableEntry* table_entry(int kind, int n, int m, int prec, const TableBuilder* build = nullptr) {
   static std::mutex mu;
   static std::map<TableKey, TableEntry> cache;
   int dev = 0;
@@ -189,7 +190,9 @@ static const TableEntry* table_entry(int kind, int n, int m, int prec) {
   if (it != cache.end()) return &it->second;
   std::vector<unsigned char> buf;
   TableEntry e;
-  if (kind == 2) {
+  if (build) {
+    (*build)(buf);
+  } else if (kind == 2) {
     push_bluestein(buf, n, m, prec, e.off[0], e.off[1], e.off[2]);
   } else if (kind == 3) {  // finite-difference factors of order m
     buf.resize((size_t)n * sizeof(double));
@@ -237,6 +240,11 @@ long double fd_factor_ld(long long k, long long n, int order) {
 const double* table_symbol(int n, int order) {
   const TableEntry* e = table_entry(3, n, order, 0);
   return e ? static_cast<const double*>(e->mem) : nullptr;
+}
+
+const void* table_built(int kind, int n, int prec, const TableBuilder& build) {
+  const TableEntry* e = table_entry(kind, n, 0, prec, &build);
+  return e ? e->mem : nullptr;
 }
 
 const void* table_twiddle(int n, int prec) {

@@ -221,6 +221,41 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     }
   }
 
+  // Mixed-radix passes: every length with a prime factor above 5 that has such a
+  // plan, and odd-length rows (in pairs), unless tuned by hand.  The four-step
+  // y order is the register engine's alone, and a plain FP32 solve (no
+  // refinement) stays on it whole: its result carries the rounding of the FP32
+  // passes, so other butterflies would move it by 4e-7, where a refined or FP64
+  // one moves by its last digits.
+  // One box, register engine and here: 385x301x338 FP64 2.98 and 1.04 ms,
+  // 131x97x150 FP32 + 2 steps 0.71 and 0.48 ms.
+  for (int prec = 0; prec < nprec; ++prec) {
+    if (prec && !o.refine_steps) continue;
+    int uE, uT, uF;
+    auto tuned = [&](int kind, int len) { return tune_lookup(kind, len, prec, uE, uT, uF); };
+    auto smooth = [](int m) {
+      for (int q : {2, 3, 5})
+        while (m % q == 0) m /= q;
+      return m == 1;
+    };
+    const int M = n[2] % 2 ? n[2] : n[2] / 2;
+    // (odd nz: the pairs of a plane are indexed below 2^16)
+    if (!p->fz.n && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
+        !(mix_cfg(M, prec, 0, n[1], n[2] % 2, p->mzr[prec]) && mix_cfg(M, prec, 3, n[1], n[2] % 2, p->mzi[prec])))
+      p->mzr[prec].plan = p->mzi[prec].plan = nullptr;
+    const bool pen = p->pencil && prec == mainp;
+    if (!p->fy.n && !smooth(n[1]) && !tuned(1, n[1])) mix_cfg(n[1], prec, 1, pen ? std::max(p->nh, n[0]) : p->nh, false, p->my[prec]);
+    if (!p->fx.n && !p->fy.n && !smooth(n[0]) && !tuned(2, n[0])) mix_cfg(n[0], prec, 2, pen ? n[1] : p->nh, false, p->mx[prec]);
+    // one workgroup per tile of a 32-bit grid
+    auto fits = [&](MixCfg& c, long long planes, long long lines) {
+      if (c.plan && planes * ((lines + c.T - 1) / c.T) > INT_MAX) c.plan = nullptr;
+    };
+    fits(p->mzr[prec], 1, (long long)n[0] * n[1]);
+    fits(p->mzi[prec], 1, (long long)n[0] * n[1]);
+    fits(p->my[prec], std::max(n[0], p->nh), std::max(n[0], p->nh));
+    fits(p->mx[prec], std::max(n[1], p->nh), std::max(n[1], p->nh));
+  }
+
   // pencil layout: the z inverse reads its rows from [i][kh][j], T
   // consecutive j per kh, so it takes 128 bytes of rows per workgroup (8
   // FP64 or 16 FP32 rows) where two such workgroups fit a CU's LDS, else 64
@@ -587,6 +622,22 @@ static RowArgs zlone_args(const ff_plan* p, int prec, const void* src, void* dst
   return a;
 }
 
+// A row pass through the mixed-radix kernels.
+static Launch mix_rows(const ff_plan* p, const MixCfg& c, RowArgs& a, hipStream_t s) {
+  a.mix = c.plan;
+  a.tw = c.tw;
+  a.T = c.T;
+  a.lgT = c.lgT;
+  a.pitch = mix_row_pitch(c.n);
+  const uint64_t per = p->n[2] % 2 ? p->nh : c.n / 2 + 1;
+  a.Linv = per > 1 ? (uint32_t)(((1ull << 32) + per - 1) / per) : 0u;
+  const uint64_t hy = (a.ny + 1) / 2;
+  a.hyinv = hy > 1 ? (uint32_t)(((1ull << 32) + hy - 1) / hy) : 0u;
+  a.nlines = p->n[2] % 2 ? a.nrows / a.ny * ((a.ny + 1) / 2) : a.nrows;
+  a.nblocks = (int)((a.nlines + c.T - 1) / c.T);
+  return Launch{dim3(a.nblocks), dim3(kMixThreads), c.lds, s};
+}
+
 // The buffers of a four-step z pass must differ, except where noted.
 static ff_status check_zfour(const ff_plan* p, long long nrows, std::initializer_list<const void*> distinct) {
   if (nrows >= 0) return set_error(FF_ERR_INVALID, "z rows in four steps: whole passes only");
@@ -708,6 +759,10 @@ ff_status run_zfwd(const ff_plan* p, int prec, int in_f32, const void* src, void
   }
   a.src = static_cast<const unsigned char*>(src) + row0 * p->n[2] * (in_f32 ? 4 : 8);
   a.dst = static_cast<unsigned char*>(dst) + row0 * p->nh * (prec ? 8 : 16);
+  if (p->mzr[prec].plan) {
+    const Launch l = mix_rows(p, p->mzr[prec], a, s);
+    return hip_check(launch_r2c(1, prec, in_f32, p->n[2] % 2, 0, 0, l, a), "z forward launch");
+  }
   const Launch l{dim3(a.nblocks), dim3(c.threads), c.lds, s};
   return hip_check(launch_r2c(c.line.E, prec, in_f32, p->n[2] % 2, c.line.bluestein(), c.stat, l, a), "z forward launch");
 }
@@ -738,6 +793,10 @@ ff_status run_zinv(const ff_plan* p, int prec, int out_kind, int epi, const void
     a.shiftp = shiftp;
     a.shift = a.scale;  // shift = (sum of phi) / N
   }
+  if (p->mzi[prec].plan) {
+    const Launch l = mix_rows(p, p->mzi[prec], a, s);
+    return hip_check(launch_c2r(1, prec, out_kind, p->n[2] % 2, epi, 0, 0, l, a), "z inverse launch");
+  }
   const RowCfg& c = p->zi[prec];
   const Launch l{dim3(a.nblocks), dim3(c.threads), c.lds, s};
   return hip_check(launch_c2r(c.line.E, prec, out_kind, p->n[2] % 2, epi, c.line.bluestein(), c.stat, l, a),
@@ -755,10 +814,12 @@ struct SubLines {
 };
 
 // One column pass launch with line configuration c (engine twiddles tw,
-// Bluestein tables bl); sub: four-step geometry (null: whole lines).
+// Bluestein tables bl); sub: four-step geometry (null: whole lines); mix: the
+// mixed-radix tile that runs it instead (null: none).
 static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, const void* src, void* dst,
                              hipStream_t s, double* dc_out, int lay_in, int lay_out, int outer0, int nouter,
-                             const ColCfg& c, const void* tw, const void* const* bl, const SubLines* sub) {
+                             const ColCfg& c, const void* tw, const void* const* bl, const SubLines* sub,
+                             const MixCfg* mix = nullptr) {
   if (src == dst && lay_in != lay_out) return set_error(FF_ERR_INVALID, "in-place column pass must keep its layout");
   if (mode == COL_FILTER && p->sym) mode = COL_FILTER_FD;
   if (mode == COL_SYMBOL && p->sym)
@@ -826,7 +887,7 @@ static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, con
   // odd nh): shift each plane's tiles onto the 64-byte grid of its rows.  The
   // tile count covers the shift.
   a.cshift_mask = a.cshift_mul = 0;
-  if (c.stat) {
+  if (c.stat && !mix) {
     const long long mask = prec ? 7 : 3;  // complex elements per 64 bytes, minus one
     const long long W = a.out.Wlast;
     if (a.in.nb == 1 && a.out.nb == 1 && ((a.out.fr * W) & mask) == 0 && ((a.out.fo * W) & mask) != 0) {
@@ -860,6 +921,17 @@ static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, con
   a.chirp = bl[0];
   a.bsf = bl[1];
   a.bsi = bl[2];
+  if (mix) {
+    a.mix = mix->plan;
+    a.tw = mix->tw;
+    a.T = mix->T;
+    a.lgT = mix->lgT;
+    a.nbuf = mix->bufs;
+    a.tiles = (a.ncols + a.T - 1) / a.T;
+    a.nblocks = a.nouter * a.tiles;  // bounded at plan creation
+    const Launch l{dim3(a.nblocks), dim3(kMixThreads), mix->lds, s};
+    return hip_check(launch_col(1, prec, mode, 0, 1, 0, 0, l, a), "column pass launch");
+  }
   // kernels with LDS twiddles also copy the x axis's finite-difference
   // factors to LDS, after the twiddles
   const size_t lds = c.lds + (mode == COL_FILTER_FD && c.stat == 2 ? (size_t)c.line.lp.n * sizeof(double) : 0);
@@ -885,7 +957,7 @@ ff_status run_col(const ff_plan* p, int prec, int axis, int mode, const void* sr
     const ColCfg& c = axis == 1 ? p->cy[prec] : p->cx[prec];
     return run_col_cfg(p, prec, axis, mode, src, dst, s, dc_out, lay_in, lay_out, outer0, nouter, c,
                        axis == 1 ? p->tw_y[prec] : p->tw_x[prec], axis == 1 ? p->bl_y[prec] : p->bl_x[prec],
-                       nullptr);
+                       nullptr, (axis == 1 ? p->my[prec] : p->mx[prec]).plan ? &(axis == 1 ? p->my : p->mx)[prec] : nullptr);
   }
   if (lay_in != LAY_PLAIN || lay_out != LAY_PLAIN || nouter >= 0)
     return set_error(FF_ERR_INVALID, "four-step column lines run over whole passes in the plain layout");

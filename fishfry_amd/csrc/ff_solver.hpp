@@ -2,6 +2,7 @@
 #pragma once
 
 #include "ff_internal.hpp"
+#include "ff_mixed.hpp"
 
 struct ff_plan {
   int n[3];
@@ -26,6 +27,9 @@ struct ff_plan {
   ff::RowCfg zr[2];  // z forward rows
   ff::RowCfg zi[2];  // z inverse rows
   ff::ColCfg cy[2], cx[2];
+  // passes of lengths the register engine would take through Bluestein, and
+  // odd-length rows (ff_mixed.hpp); plan null: the configurations above
+  ff::MixCfg mzr[2], mzi[2], my[2], mx[2];
   const void* tw_z[2];   // z forward engine twiddles
   const void* tw_zi[2];  // z inverse engine twiddles (its E, hence m, may differ)
   const void* tw_zpost[2];
