@@ -141,8 +141,15 @@ ff_status prepare_groups(ff_batch* b, double* const* d, double* const* p) {
   std::vector<std::vector<PassLaunch>> rec(b->count);
   for (int i = 0; i < b->count; ++i) {
     if (solo(b, i)) continue;
+    // (the group's instances fill the chip together)
+    int same = 0;
+    for (int k = 0; k < b->count; ++k)
+      same += std::equal(b->items[k].n, b->items[k].n + 3, b->items[i].n) &&
+              b->items[k].precision == b->items[i].precision && b->items[k].refine_steps == b->items[i].refine_steps;
+    ff_plan plan = *b->plans[i];
+    plan_choose_planes(&plan, same);
     set_launch_recorder(&rec[i]);
-    const ff_status st = solve_enqueue(b->plans[i], d[i], p[i], nullptr, nullptr);
+    const ff_status st = solve_enqueue(&plan, d[i], p[i], nullptr, nullptr);
     set_launch_recorder(nullptr);
     if (st != FF_OK) return st;
   }
@@ -305,7 +312,9 @@ ff_status prepare_steps(ff_batch* b, double* const* d, double* const* p) {
   for (int i = 0; i < b->count; ++i) {
     if (solo(b, i)) continue;
     set_launch_recorder(&rec[i]);
-    const ff_status st = solve_enqueue(b->plans[i], d[i], p[i], nullptr, nullptr);
+    ff_plan plan = *b->plans[i];  // the passes one by one: plane kernels have no multi-shape variant
+    plan.plane[0] = plan.plane[1] = 0;
+    const ff_status st = solve_enqueue(&plan, d[i], p[i], nullptr, nullptr);
     set_launch_recorder(nullptr);
     if (st != FF_OK) return st;
   }
@@ -678,6 +687,8 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
         // nor have mixed-radix ones
         const MixCfg* mix[4] = {&p->mzr[prec], &p->my[prec], &p->mx[prec], &p->mzi[prec]};
         if (mix[kv[0]]->plan) continue;
+        // z and y passes that run as plane kernels stay so
+        if (p->plane[prec] && kv[0] != 2) continue;
         if (!seen.count({kv[0], kv[1], prec})) seen[{kv[0], kv[1], prec}] = i;
       }
     }

@@ -5,6 +5,7 @@
 
 #include "ff_kernels.hpp"
 #include "ff_mixed.hpp"
+#include "ff_plane.hpp"
 
 #ifndef FF_E
 #error "FF_E must be defined"
@@ -102,7 +103,8 @@ static const void* col_static_fn(int f32, int split, int mode, int n, int T, int
 }
 
 // Bluestein lines use the default kernel shape (one group, complex exchange).
-// Mixed-radix passes (a.mix) have no elements per thread: they dispatch as E = 1.
+// Mixed-radix passes (a.mix) and plane kernels (a.plane) have no elements per
+// thread of their own: they dispatch as E = 1.
 template <>
 hipError_t PassLaunchers<FF_E>::col(int f32, int mode, int split, int groups, int blue, int stat, const Launch& l,
                                     const ColArgs& a) {
@@ -161,7 +163,10 @@ template <>
 hipError_t PassLaunchers<FF_E>::r2c(int f32, int in_f32, int odd, int blue, int stat, const Launch& l,
                                     const RowArgs& a) {
   if constexpr (FF_E == 1)
+  {
     if (a.mix) return mix_r2c(f32, in_f32, odd, l, a);
+    if (a.plane) return plane_r2c(f32, in_f32, l, a);
+  }
   const void* fn = stat ? r2c_static_fn<0>(f32, in_f32, odd, a.lp.n, stat)
                         : (blue ? r2c_fn<true>(f32, in_f32, odd) : r2c_fn<false>(f32, in_f32, odd));
   if (!fn) return hipErrorInvalidValue;
@@ -212,7 +217,10 @@ template <>
 hipError_t PassLaunchers<FF_E>::c2r(int f32, int out_kind, int odd, int epi, int blue, int stat, const Launch& l,
                                     const RowArgs& a) {
   if constexpr (FF_E == 1)
+  {
     if (a.mix) return mix_c2r(f32, out_kind, odd, epi, l, a);
+    if (a.plane) return plane_c2r(f32, out_kind, epi, l, a);
+  }
   const void* fn = stat ? c2r_static_fn<0>(f32, out_kind, odd, epi, a.lp.n, stat)
                         : (blue ? c2r_fn<true>(f32, out_kind, odd, epi) : c2r_fn<false>(f32, out_kind, odd, epi));
   if (!fn) return hipErrorInvalidValue;

@@ -581,6 +581,8 @@ struct RowArgs {
   long long nlines;               // mixed-radix pass: lines (rows, or for odd nz pairs of them);
   int lgT;                        // T = 2^lgT; Linv = ceil(2^32 / half-spectrum steps per line) and
   uint32_t hyinv;                 // ceil(2^32 / pairs per plane)
+  const void* tw2;                // plane kernels: the column twiddles
+  int plane;                      // the z and y passes of whole planes (ff_plane.hpp)
   int m1;                         // four-step z rows: the stride-1 sub-line length (ff_zsplit.hip)
   int lone;                       // odd nz, nx*ny odd: the launch's one pair is the last row alone
                                   // (no second row: zero on the way in, not written on the way out)

@@ -6,7 +6,7 @@
 // MB: 0.11 ms at the rate of the row kernels): Bluestein's lines were bound by
 // their four transforms of at least twice the length and by the registers of
 // the kernels that hold them (x 1.27 ms, y 0.32, z forward 0.50, z inverse 0.61);
-// here x takes 0.27 ms, y 0.22, z 0.15 and 0.17, bound by the LDS exchanges and
+// here x takes 0.31 ms, y 0.22, z 0.18 and 0.20, bound by the LDS exchanges and
 // index arithmetic of the stages.  A tile is about 2048 FP64 (4096 FP32) values,
 // 32 to 50 KB of LDS in two buffers, so three or four workgroups of 256 threads
 // share a CU and one's memory phase covers another's stages; columns keep

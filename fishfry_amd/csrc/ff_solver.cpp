@@ -275,6 +275,19 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     }
   }
 
+  // Planes that fit a CU: their z and y passes as one kernel each way, where the
+  // passes would run the same plans in the plain layout.
+  for (int prec = 0; prec < nprec; ++prec) {
+    int uE, uT, uF;
+    const int kz = plane_index(n[2]), ky = plane_index(n[1]);
+    p->planes_fit[prec] =
+        kz >= 0 && ky >= 0 && plane_threads(n[2], n[1]) > 0 && !p->pencil && !p->lgKT && !p->slab && !four &&
+        p->zr[prec].line.E == kPlaneLens[kz].ez && p->zi[prec].line.E == kPlaneLens[kz].ez &&
+        p->cy[prec].line.E == kPlaneLens[ky].ey && !tune_lookup(0, n[2] / 2, prec, uE, uT, uF) &&
+        !tune_lookup(3, n[2] / 2, prec, uE, uT, uF) && !tune_lookup(1, n[1], prec, uE, uT, uF);
+  }
+  plan_choose_planes(p, 1);
+
   // one workgroup per tile: every pass's grid must fit a 32-bit grid size
   for (int prec = 0; prec < nprec; ++prec) {
     const long long rows = (long long)n[0] * n[1];
@@ -371,6 +384,18 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
   }
   *out = p;
   return FF_OK;
+}
+
+// Whether the plane kernels run a plan's z and y passes, with `instances` solves
+// of it in one launch: always for planes of up to 6144 points, several of which
+// share a CU; larger ones take a CU each, and then need enough of them.  (One
+// box, passes and planes: 64^3 FP64 21.3 and 17.8 us; 32x96x32 29 and 17;
+// 1000x64x64 82 and 62; 32x128x128 28 and 38; 256x128x128 74 and 60; FP32
+// 128x128x128 37 and 38, 256x128x128 80 and 60.)
+void plan_choose_planes(ff_plan* p, int instances) {
+  const long long planes = (long long)p->n[0] * instances;
+  for (int prec = 0; prec < 2; ++prec)
+    p->plane[prec] = p->planes_fit[prec] && ((long long)p->n[1] * p->n[2] <= 6144 || planes >= (prec ? 192 : 128));
 }
 
 static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
@@ -803,6 +828,37 @@ ff_status run_zinv(const ff_plan* p, int prec, int out_kind, int epi, const void
                    "z inverse launch");
 }
 
+// The z and y passes of every plane (p->plane): forward (z, then y) from the
+// real rows src to the spectrum dst, inverse (y, then z and the epilogue) back.
+// src and dst must not overlap: a plane's rows and its spectrum differ in size.
+static ff_status run_planes_fwd(const ff_plan* p, int prec, int in_f32, const void* src, void* dst, hipStream_t s) {
+  RowArgs a = row_args(p, prec, false);
+  a.src = src;
+  a.dst = dst;
+  a.plane = 1;
+  a.tw2 = p->tw_y[prec];
+  a.nblocks = p->n[0];
+  const Launch l{dim3(a.nblocks), dim3(plane_threads(a.nz, a.ny)), plane_lds(a.nz, a.ny, prec), s};
+  return hip_check(launch_r2c(1, prec, in_f32, 0, 0, 0, l, a), "plane forward launch");
+}
+
+static ff_status run_planes_inv(const ff_plan* p, int prec, int out_kind, int epi, const void* src, void* dst,
+                                const double* f, const double* shiftp, hipStream_t s) {
+  RowArgs a = row_args(p, prec, true);
+  a.src = src;
+  a.dst = dst;
+  a.aux = f;
+  if (shiftp) {
+    a.shiftp = shiftp;
+    a.shift = a.scale;  // shift = (sum of phi) / N
+  }
+  a.plane = 1;
+  a.tw2 = p->tw_y[prec];
+  a.nblocks = p->n[0];
+  const Launch l{dim3(a.nblocks), dim3(plane_threads(a.nz, a.ny)), plane_lds(a.nz, a.ny, prec), s};
+  return hip_check(launch_c2r(1, prec, out_kind, 0, epi, 0, 0, l, a), "plane inverse launch");
+}
+
 // Plane and position geometry of a four-step sub-line pass (plain layout, in
 // rows of nh): planes (lo, hi) with lo < nlo, strides fo (lo), fo2 (hi) and
 // fr (positions); the W_n twiddle and the x filter's i map.
@@ -1003,6 +1059,11 @@ static ff_status fp32_round_trip(const ff_plan* p, int in_f32, const void* src, 
   void* a = p->spec;
   void* b = p->pencil ? static_cast<void*>(static_cast<char*>(p->spec) + p->Nh * 8) : p->spec;
   ff_status st;
+  if (p->plane[1]) {
+    if ((st = run_planes_fwd(p, 1, in_f32, src, a, s))) return st;
+    if ((st = run_col(p, 1, 0, COL_FILTER, a, a, s, dc_col))) return st;
+    return run_planes_inv(p, 1, 0, epi, a, phi, nullptr, shiftp, s);
+  }
   if ((st = run_zfwd(p, 1, in_f32, src, a, s))) return st;
   if (p->pencil) {
     if ((st = run_col(p, 1, 1, COL_FWD, a, b, s, nullptr, LAY_PLAIN, LAY_D))) return st;
@@ -1030,13 +1091,22 @@ static ff_status solve_fp32_refine(const ff_plan* p, const double* f, double* ph
     } else {
       // r = f - L_h phi in FP64, with the same spectral symbol the filter inverts;
       // the x pass also captures sum(phi) for the FP64 mean removal
-      if ((st = run_zfwd(p, 0, 0, phi, spec, s))) return st;
-      if ((st = run_col(p, 0, 1, COL_FWD, spec, spec, s))) return st;
+      if (p->plane[0]) {
+        if ((st = run_planes_fwd(p, 0, 0, phi, spec, s))) return st;
+      } else {
+        if ((st = run_zfwd(p, 0, 0, phi, spec, s))) return st;
+        if ((st = run_col(p, 0, 1, COL_FWD, spec, spec, s))) return st;
+      }
       if ((st = run_col(p, 0, 0, COL_SYMBOL, spec, spec, s, p->dc))) return st;
-      if ((st = run_col(p, 0, 1, COL_INV, spec, spec, s))) return st;
       // r = (f - mean f) - L_h phi: L_h phi has no mean, and removing f's mean
       // keeps the FP32 rounding of r relative to the residual itself
-      if ((st = run_zinv(p, 0, 1, EPI_RESIDUAL, spec, p->res, f, p->dcf, s))) return st;
+      if (p->plane[0]) {
+        st = run_planes_inv(p, 0, 1, EPI_RESIDUAL, spec, p->res, f, p->dcf, s);
+      } else {
+        if ((st = run_col(p, 0, 1, COL_INV, spec, spec, s))) return st;
+        st = run_zinv(p, 0, 1, EPI_RESIDUAL, spec, p->res, f, p->dcf, s);
+      }
+      if (st) return st;
     }
     // correction in FP32: phi += L_h^-1 r - mean(phi)
     if ((st = fp32_round_trip(p, 1, p->res, phi, EPI_ACCUM, nullptr, p->dc, s))) return st;
@@ -1084,6 +1154,19 @@ ff_status solve_enqueue(const ff_plan* p, double* density, double* potential, hi
     }
     if (ev && (st = hip_check(hipEventRecord(ev[3], s), "event"))) return st;
     if (ev && (st = hip_check(hipEventRecord(ev[4], s), "event"))) return st;
+    return FF_OK;
+  }
+  if (p->plane[0]) {
+    // (the spectrum must leave potential before its planes are overwritten by
+    // real rows: the x pass moves it to w)
+    if ((st = run_planes_fwd(p, 0, 0, density, potential, s))) return st;
+    for (int e = 0; e < 2; ++e)
+      if (ev && (st = hip_check(hipEventRecord(ev[e], s), "event"))) return st;
+    if ((st = run_col(p, 0, 0, COL_FILTER, potential, w, s))) return st;
+    if (ev && (st = hip_check(hipEventRecord(ev[2], s), "event"))) return st;
+    if ((st = run_planes_inv(p, 0, 0, EPI_STORE, w, potential, nullptr, nullptr, s))) return st;
+    for (int e = 3; e < 5; ++e)
+      if (ev && (st = hip_check(hipEventRecord(ev[e], s), "event"))) return st;
     return FF_OK;
   }
   if ((st = run_zfwd(p, 0, 0, density, potential, s))) return st;

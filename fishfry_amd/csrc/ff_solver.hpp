@@ -3,6 +3,7 @@
 
 #include "ff_internal.hpp"
 #include "ff_mixed.hpp"
+#include "ff_plane.hpp"
 
 struct ff_plan {
   int n[3];
@@ -30,6 +31,9 @@ struct ff_plan {
   // passes of lengths the register engine would take through Bluestein, and
   // odd-length rows (ff_mixed.hpp); plan null: the configurations above
   ff::MixCfg mzr[2], mzi[2], my[2], mx[2];
+  // the z and y passes of whole planes run as one (ff_plane.hpp)
+  int plane[2];
+  int planes_fit[2];  // whether they can (plan_choose_planes decides)
   const void* tw_z[2];   // z forward engine twiddles
   const void* tw_zi[2];  // z inverse engine twiddles (its E, hence m, may differ)
   const void* tw_zpost[2];
@@ -107,6 +111,7 @@ ff_status solve_enqueue(const ff_plan* p, double* density, double* potential, hi
 ff_status plan_create(const int n[3], const double lo[3], const double hi[3], const ff_options* opts,
                       ff_plan** out, bool own_scratch = true);
 void plan_destroy(ff_plan* p);
+void plan_choose_planes(ff_plan* p, int instances);
 // Whether an FP64 grid of extents n runs its z rows in four steps, which
 // needs the work array (z_work_bytes; the plan's own unless created with
 // own_scratch false).
