@@ -231,7 +231,7 @@ bool groups_current(const ff_batch* b, double* const* d, double* const* p) {
 // LDS bytes.
 bool col_desc(const PassLaunch& r, MultiColDesc& out, size_t& lds) {
   const ColArgs& c = r.col;
-  if (r.blue || r.groups != 1 || r.split || c.outer_fast) return false;
+  if (r.blue || r.groups != 1 || (r.split && r.stat != kLdsStat) || c.outer_fast) return false;
   if (c.in.nlo || c.xtw || c.imap_n2 || c.jmap_n1) return false;  // four-step lines
   if (c.mix) return false;                                        // mixed-radix lines
   if (c.in.nb != 1 || c.out.nb != 1 || c.in.lgKT < 30 || c.out.lgKT < 30 || c.nline != c.lp.n) return false;
@@ -703,6 +703,27 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
     // column passes: split exchange, two groups, and (flags 4) the generic
     // kernel where one with the line plan compiled in exists
     const int nflags = (kind == 1 || kind == 2) ? 5 : 1;
+    double* src = density[kv.second];
+    double* dst = potential[kv.second];
+    auto time_pass = [&](const ff_plan& trial, double& ms) -> ff_status {
+      auto launch = [&]() -> ff_status {
+        if (kind == 0) return run_zfwd(&trial, prec, 0, src, dst, s);
+        if (kind == 3) return run_zinv(&trial, prec, 0, EPI_STORE, src, dst, nullptr, nullptr, s);
+        return run_col(&trial, prec, kind == 1 ? 1 : 0, kind == 2 ? COL_FILTER : COL_FWD, src, dst, s);
+      };
+      ff_status r = launch();
+      if (r == FF_OK) r = hip_check(hipEventRecord(e0, s), "event");
+      for (int k = 0; k < reps && r == FF_OK; ++k) r = launch();
+      if (r == FF_OK) r = hip_check(hipEventRecord(e1, s), "event");
+      if (r == FF_OK) r = hip_check(hipEventSynchronize(e1), "event sync");
+      float t = 0.f;
+      if (r == FF_OK) r = hip_check(hipEventElapsedTime(&t, e0, e1), "elapsed");
+      ms = t;
+      return r;
+    };
+    // the plan's own configuration (which may be a kernel that no override selects)
+    // stays unless a candidate beats it
+    st = time_pass(*p, best);
     for (int E : kEValues) {
       for (int cand = 0; cand < 7 * nflags && st == FF_OK; ++cand) {
         const int T = 1 << (cand % 7);
@@ -721,21 +742,8 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
           if (ok) (kind == 1 ? trial.cy : trial.cx)[prec] = c;
         }
         if (!ok) continue;
-        const int ip = kv.second;
-        double* src = density[ip];
-        double* dst = potential[ip];
-        auto launch = [&]() -> ff_status {
-          if (kind == 0) return run_zfwd(&trial, prec, 0, src, dst, s);
-          if (kind == 3) return run_zinv(&trial, prec, 0, EPI_STORE, src, dst, nullptr, nullptr, s);
-          return run_col(&trial, prec, kind == 1 ? 1 : 0, kind == 2 ? COL_FILTER : COL_FWD, src, dst, s);
-        };
-        st = launch();
-        if (st == FF_OK) st = hip_check(hipEventRecord(e0, s), "event");
-        for (int r = 0; r < reps && st == FF_OK; ++r) st = launch();
-        if (st == FF_OK) st = hip_check(hipEventRecord(e1, s), "event");
-        if (st == FF_OK) st = hip_check(hipEventSynchronize(e1), "event sync");
-        float ms = 0.f;
-        if (st == FF_OK) st = hip_check(hipEventElapsedTime(&ms, e0, e1), "elapsed");
+        double ms = 0.0;
+        st = time_pass(trial, ms);
         if (st == FF_OK && ms < best) {
           best = ms;
           bE = E;
@@ -747,8 +755,8 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
     if (st == FF_OK && bE) {
       const ff_tune t{kind, n, prec, bE, bT, bF};
       st = tune_set(&t);
-      count++;
     }
+    if (st == FF_OK) count++;
   }
   if (st == FF_OK) {
     drop_graph(b);

@@ -253,12 +253,16 @@ template <typename F>
 __device__ __forceinline__ cx<F> tw_at(const cx<F>* __restrict__ tw, int t) {
   return tw[t];
 }
-// The first half of a table of even length 2H, held in LDS by the kernel:
+// The first H entries of a table, held in LDS by the kernel: the whole of an odd
+// length, the first half of an even one, for which
 // W[t + H] = -W[t] exactly in the host's tables (a half turn adds two quarter
 // turns to the same reduced angle, so only the signs differ), so the negated
 // entry is bit-identical to the stored one.  Entry t is stored at
 // tw_swizzle(t): a permutation within blocks of 16 entries that spreads the
-// strided indices of a wave's lanes (t = m*k*twstep) over the LDS banks.
+// strided indices of a wave's lanes (t = m*k*twstep) over the LDS banks (so
+// the table takes whole blocks).
+__host__ __device__ constexpr int tw_lds_entries(int n) { return n % 2 ? n : n / 2; }
+__host__ __device__ constexpr int tw_lds_slots(int n) { return (tw_lds_entries(n) + 15) / 16 * 16; }
 __device__ __forceinline__ int tw_swizzle(int t) { return t ^ (((t >> 4) ^ (t >> 8)) & 15); }
 template <typename F, int H>
 struct TwHalf {

@@ -111,7 +111,9 @@ hipError_t PassLaunchers<FF_E>::col(int f32, int mode, int split, int groups, in
   const void* fn = nullptr;
   if constexpr (FF_E == 1)
     if (a.mix) return mix_col(f32, mode, l, a);
-  if (stat) {
+  if (stat == kLdsStat) {
+    fn = lds_col_kernel(f32, mode, a.lp.n, FF_E);
+  } else if (stat) {
     fn = col_static_fn<0>(f32, split, mode, a.lp.n, a.T, stat);
   } else if (blue) {
     if (groups == 1 && !split) fn = col_fn<FF_E, false, 1, true>(f32, mode);
@@ -167,7 +169,8 @@ hipError_t PassLaunchers<FF_E>::r2c(int f32, int in_f32, int odd, int blue, int 
     if (a.mix) return mix_r2c(f32, in_f32, odd, l, a);
     if (a.plane) return plane_r2c(f32, in_f32, l, a);
   }
-  const void* fn = stat ? r2c_static_fn<0>(f32, in_f32, odd, a.lp.n, stat)
+  const void* fn = stat == kLdsStat ? lds_r2c_kernel(f32, in_f32, odd, a.lp.n, FF_E)
+                   : stat ? r2c_static_fn<0>(f32, in_f32, odd, a.lp.n, stat)
                         : (blue ? r2c_fn<true>(f32, in_f32, odd) : r2c_fn<false>(f32, in_f32, odd));
   if (!fn) return hipErrorInvalidValue;
   return launch(fn, l, &a, sizeof(a));
@@ -221,7 +224,8 @@ hipError_t PassLaunchers<FF_E>::c2r(int f32, int out_kind, int odd, int epi, int
     if (a.mix) return mix_c2r(f32, out_kind, odd, epi, l, a);
     if (a.plane) return plane_c2r(f32, out_kind, epi, l, a);
   }
-  const void* fn = stat ? c2r_static_fn<0>(f32, out_kind, odd, epi, a.lp.n, stat)
+  const void* fn = stat == kLdsStat ? lds_c2r_kernel(f32, out_kind, odd, epi, a.lp.n, FF_E)
+                   : stat ? c2r_static_fn<0>(f32, out_kind, odd, epi, a.lp.n, stat)
                         : (blue ? c2r_fn<true>(f32, out_kind, odd, epi) : c2r_fn<false>(f32, out_kind, odd, epi));
   if (!fn) return hipErrorInvalidValue;
   return launch(fn, l, &a, sizeof(a));

@@ -82,7 +82,8 @@ struct ColCfg {
   int split = 0;   // FF_TUNE_SPLIT_LDS: one component per LDS slot
   int groups = 1;  // FF_TUNE_TWO_GROUPS: column groups of T per workgroup
   int stat = 0;    // a kStaticCols kernel runs this configuration (FF_TUNE_GENERIC clears it):
-                   // 1 twiddles from the table in memory, 2 from LDS (FF_TUNE_LDS_TWIDDLES)
+                   // 1 twiddles from the table in memory, 2 from LDS (FF_TUNE_LDS_TWIDDLES),
+                   // kLdsStat a kLdsCols kernel
   size_t lds = 0;
   int threads = 0;
 };
@@ -94,7 +95,8 @@ struct RowCfg {
   int threads = 0;
   uint32_t Linv = 0;
   int stat = 0;  // a kStaticRows kernel runs this configuration (FF_TUNE_GENERIC clears it);
-                 // 2: the one that reads its twiddles from LDS (FF_TUNE_LDS_TWIDDLES)
+                 // 2: the one that reads its twiddles from LDS (FF_TUNE_LDS_TWIDDLES);
+                 // kLdsStat a kLdsRows kernel
 };
 
 // kind: 0 z forward rows, 1 y columns, 2 x columns, 3 z inverse rows;
@@ -106,6 +108,11 @@ bool make_col_cfg(int n, int ncols, int elem_bytes, ColCfg& out, int kind, int p
 bool make_row_cfg(int nz, int elem_bytes, RowCfg& out, int kind, int prec);
 bool col_cfg_with(int n, int ncols, int elem_bytes, ColCfg& out, int E, int T, int flags, int kind);
 bool row_cfg_with(int nz, int elem_bytes, RowCfg& out, int E, int T, int flags);
+// A plan's configuration with the line plan compiled in and twiddles in LDS, in place of
+// a default one (the same elements per thread, hence the same results to the bit);
+// unchanged where there is no such kernel.
+void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind);
+void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes);
 bool tune_lookup(int kind, int n, int prec, int& E, int& T, int& flags);
 ff_status tune_set(const ff_tune* t);
 void tune_reset();

@@ -278,7 +278,7 @@ __device__ __forceinline__ void col_line(cx<F> (&v)[E], const ColArgs& a, const 
         const int ii = plo + istep * (r0 + i * L);
         double gi;
         if constexpr (is_tw_half<TW>::value)
-          gi = reinterpret_cast<const double*>(tw.p + SN / 2)[ii];  // LDS copy (compiled-in: ii < SN = nx)
+          gi = reinterpret_cast<const double*>(tw.p + tw_lds_slots(SN))[ii];  // LDS copy (compiled-in: ii < SN = nx)
         else
           gi = glb<const double>(a.symx)[ii < a.nx ? ii : 0];
         const double s2 = fmadd(gk, io.ddk, fmadd(gi, io.ddi, tj));  // (i + j) + k
@@ -436,9 +436,9 @@ __device__ __forceinline__ void col_transform(cx<F> (&v)[G][E], const ColArgs& a
   int c, r0;
   col_thread<E, SN, ST>(a, c, r0);
   if constexpr (TWL) {
-    static_assert(SN > 0 && SN % 32 == 0, "LDS twiddles: compiled-in plans, length a multiple of 32");
+    static_assert(SN > 0, "LDS twiddles: compiled-in plans");
     const ColIdx idx{T, c, kColPadShift};
-    const TwHalf<F, SN / 2> tw{reinterpret_cast<const cx<F>*>(smem_raw + col_exchange_bytes<F, SPLIT, SN, ST>())};
+    const TwHalf<F, tw_lds_entries(SN)> tw{reinterpret_cast<const cx<F>*>(smem_raw + col_exchange_bytes<F, SPLIT, SN, ST>())};
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const int col = (t.tile * G + g) * T + c - t.sh;
@@ -486,12 +486,12 @@ __device__ __forceinline__ void col_tile(const ColArgs& a, const PassInst& io, i
   col_store<F, E, G, BL, SN, ST, MODE>(v, a, io, t);
 }
 
-// Copies the first half of the twiddle table (SN/2 entries, swizzled) to LDS
+// Copies the twiddle table (tw_lds_entries, swizzled) to LDS
 // after the exchange area, for col_transform<..., TWL = true>.  The tile's
 // loads are issued first, so the copy overlaps them.  The twiddle loads of
 // the transforms otherwise go through the vector memory path that the tile's
 // own loads and stores keep busy: from LDS the FP64 x pass at 1024 takes 7 %
-// less time on MI355X.  Launch LDS: col_exchange_bytes + (SN/2) complex values.
+// less time on MI355X.  Launch LDS: col_exchange_bytes + tw_lds_slots(SN) complex values.
 template <typename F, bool SPLIT, int SN, int ST, int THREADS, int MODE = COL_FWD>
 __device__ __forceinline__ void col_twiddles_to_lds(const ColArgs& a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -502,11 +502,12 @@ __device__ __forceinline__ void col_twiddles_to_lds(const ColArgs& a) {
   // for each load in turn, behind the tile's loads
   // (indexes clamped into the table: every load is unconditional, which
   // keeps the values in registers)
-  constexpr int NT = (SN / 2 + THREADS - 1) / THREADS;
+  constexpr int H = tw_lds_entries(SN);
+  constexpr int NT = (H + THREADS - 1) / THREADS;
   cx<F> tv[NT];
 #pragma unroll
   for (int k = 0; k < NT; ++k) {
-    const int i = min((int)threadIdx.x + k * THREADS, SN / 2 - 1);
+    const int i = min((int)threadIdx.x + k * THREADS, H - 1);
     tv[k] = cx<F>{twg[i].x, twg[i].y};
   }
   // (finite-difference x pass: the x axis's factors, SN doubles, follow the
@@ -522,10 +523,10 @@ __device__ __forceinline__ void col_twiddles_to_lds(const ColArgs& a) {
 #pragma unroll
   for (int k = 0; k < NT; ++k) {
     const int i = threadIdx.x + k * THREADS;
-    if (i < SN / 2) twl[tw_swizzle(i)] = tv[k];
+    if (i < H) twl[tw_swizzle(i)] = tv[k];
   }
   if constexpr (NS > 0) {
-    double* sym = reinterpret_cast<double*>(twl + SN / 2);
+    double* sym = reinterpret_cast<double*>(twl + tw_lds_slots(SN));
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
       const int i = threadIdx.x + k * THREADS;
@@ -605,14 +606,21 @@ __device__ __forceinline__ long long spec_row(const RowArgs& a, long long row) {
 // SN > 0: the plan of the row transform, length SN, is compiled in (even nz).
 // r2c_tile: the work of one workgroup, row block blk (< a.nblocks), with the
 // per-instance fields io (k_r2c: one pass; ff_multi.hip: many instances).
+// Waves per SIMD that the registers of a row kernel must allow: two where many elements
+// per thread would let it take them all.
+template <int E, int SN, bool TWL>
+constexpr int row_waves() {
+  return SN > 0 && TWL && E >= 20 ? 2 : 1;
+}
+
 // TWL (compiled-in plans): the first half of the W_SN table is copied to LDS
 // after the T row tiles and the passes read their twiddles there.
 template <typename F, int SN>
-__device__ __forceinline__ TwHalf<F, SN / 2> row_twiddles_to_lds(const RowArgs& a, cx<F>* lds) {
+__device__ __forceinline__ TwHalf<F, tw_lds_entries(SN)> row_twiddles_to_lds(const RowArgs& a, cx<F>* lds) {
   cx<F>* twl = lds + (long long)a.T * a.pitch;
   const cx<F>* __restrict__ twg = reinterpret_cast<const cx<F>*>(a.tw);
-  for (int i = threadIdx.x; i < SN / 2; i += blockDim.x) twl[tw_swizzle(i)] = twg[i];
-  return TwHalf<F, SN / 2>{twl};
+  for (int i = threadIdx.x; i < tw_lds_entries(SN); i += blockDim.x) twl[tw_swizzle(i)] = twg[i];
+  return TwHalf<F, tw_lds_entries(SN)>{twl};
 }
 
 template <typename F, typename IN, int E, bool ODD, bool BL, int SN, bool TWL = false>
@@ -652,7 +660,7 @@ __device__ __forceinline__ void r2c_tile(const RowArgs& a, const PassInst& io, i
     }
     if constexpr (TWL) {
       static_assert(SN > 0 && !BL, "LDS twiddles: compiled-in plans");
-      const TwHalf<F, SN / 2> twl = row_twiddles_to_lds<F, SN>(a, lds);
+      const auto twl = row_twiddles_to_lds<F, SN>(a, lds);
       __syncthreads();
       line_dft<E, -1, F, RI, false, BL, SN>(v, a.lp, M, twl, a.chirp, a.bsf, a.bsi, lds, idx, r0);
     } else {
@@ -700,7 +708,7 @@ __device__ __forceinline__ void r2c_tile(const RowArgs& a, const PassInst& io, i
 }
 
 template <typename F, typename IN, int E, bool ODD, bool BL, int SN = 0, bool TWL = false>
-__global__ __launch_bounds__(max_threads_for(E)) void k_r2c(const RowArgs a) {
+__global__ __launch_bounds__(max_threads_for(E), (row_waves<E, SN, TWL>())) void k_r2c(const RowArgs a) {
   r2c_tile<F, IN, E, ODD, BL, SN, TWL>(a, inst_of(a), xcd_remap(blockIdx.x, a.nblocks));
 }
 
@@ -825,7 +833,7 @@ __device__ __forceinline__ void c2r_tile(const RowArgs& a, const PassInst& io, i
           src[(long long)kb * a.spec.KS + r * W + kt];
     }
   }
-  TwHalf<F, (SN > 0 ? SN / 2 : 1)> twl{nullptr};
+  TwHalf<F, (SN > 0 ? tw_lds_entries(SN) : 1)> twl{nullptr};
   if constexpr (TWL) {
     static_assert(SN > 0 && !BL, "LDS twiddles: compiled-in plans");
     twl = row_twiddles_to_lds<F, SN>(a, lds);
@@ -888,7 +896,7 @@ __device__ __forceinline__ void c2r_tile(const RowArgs& a, const PassInst& io, i
 }
 
 template <typename F, typename OUT, int E, bool ODD, int EPI, bool BL, int SN = 0, bool TWL = false>
-__global__ __launch_bounds__(max_threads_for(E)) void k_c2r(const RowArgs a) {
+__global__ __launch_bounds__(max_threads_for(E), (row_waves<E, SN, TWL>())) void k_c2r(const RowArgs a) {
   c2r_tile<F, OUT, E, ODD, EPI, BL, SN, TWL>(a, inst_of(a), xcd_remap(blockIdx.x, a.nblocks));
 }
 
@@ -941,6 +949,79 @@ struct StaticRow {
 constexpr StaticRow kStaticRows[] = {{512, 8}, {500, 10}, {384, 12}, {384, 24}, {256, 16}, {128, 16}, {80, 20},
                                      {64, 8},  {48, 12},  {32, 8},   {24, 12},  {16, 16}};
 constexpr int kNumStaticRows = sizeof(kStaticRows) / sizeof(kStaticRows[0]);
+
+// Lines of every other 2^a 3^b 5^c length to 1024 (columns) and 512 (rows of nz/2), with the
+// elements per thread that the planner takes for them (built-in ones at 512, 768 and
+// 1000), compiled in with twiddles from LDS.  A plan takes these kernels where the length
+// is not tuned (col_lds_twiddles, row_lds_twiddles); the results are those of the generic
+// kernel to the bit.  What bounded the generic kernel was its own arithmetic -- positions,
+// moduli and twiddle indexes per element -- and the registers it took (two waves per SIMD
+// at most from E = 20 on), then the twiddle loads, which share the vector memory path with
+// the tile's; generic kernels with the twiddles in LDS alone were no faster.  Passes in
+// us on MI355X, generic and these (FP64; z, y, x, y inverse, z inverse):
+//   900^3  5404 4641 6543 4051 4828   3302 2515 3587 2419 3506
+//   640^3  1162 1475 2095 1338 1137    875  849 1276  843 1244
+//   240^3    97   83  138   83   83     70   50   76   48   59
+//   1000^3 3088 4426 5184 3915 3426   2908 3579 4553 3232 3291  (of them x compiled in before)
+// What bounds them now is memory: 2.4-2.5 ms is 4.8 TB/s at 900^3.
+struct LdsLine {
+  int n, E;
+};
+constexpr LdsLine kLdsCols[] = {{36, 6}, {40, 20}, {45, 15}, {50, 10}, {54, 6}, {60, 30},
+    {72, 12}, {75, 15}, {80, 20}, {81, 3}, {90, 30}, {100, 10}, {108, 6}, {120, 30}, {125, 5},
+    {135, 15}, {144, 12}, {150, 30}, {160, 20}, {162, 6}, {180, 30}, {192, 12}, {200, 10}, {216, 6},
+    {225, 15}, {240, 30}, {243, 3}, {250, 10}, {256, 16}, {270, 30}, {288, 12}, {300, 30}, {320, 20}, {324, 6},
+    {360, 30}, {375, 15}, {384, 24}, {400, 20}, {405, 15}, {432, 12}, {450, 30}, {480, 30}, {486, 6}, {500, 10},
+    {512, 8}, {540, 30}, {576, 12}, {600, 30}, {625, 5}, {640, 20}, {648, 6}, {675, 15}, {720, 30}, {729, 3},
+    {750, 30}, {768, 12}, {768, 24}, {800, 20}, {810, 30}, {864, 12}, {900, 30}, {960, 30}, {972, 6}, {1000, 10},
+    {1000, 20}};
+constexpr LdsLine kLdsRows[] = {{18, 6}, {20, 10}, {25, 5}, {27, 3}, {30, 30}, {36, 6}, {40, 20}, {45, 15},
+    {50, 10}, {54, 6}, {60, 30}, {72, 12}, {75, 15}, {81, 3}, {90, 30}, {96, 24}, {100, 10}, {108, 6}, {120, 30},
+    {125, 5}, {135, 15}, {144, 12}, {150, 30}, {160, 20}, {162, 6}, {180, 30}, {192, 12}, {200, 10}, {216, 6},
+    {225, 15}, {240, 30}, {243, 3}, {250, 10}, {270, 30}, {288, 12}, {300, 30}, {320, 20}, {324, 6}, {360, 30},
+    {375, 15}, {400, 20}, {405, 15}, {432, 12}, {450, 30}, {480, 30}, {486, 6}};
+constexpr int kNumLdsCols = sizeof(kLdsCols) / sizeof(kLdsCols[0]);
+constexpr int kNumLdsRows = sizeof(kLdsRows) / sizeof(kLdsRows[0]);
+// stat of these kernels, and the kernels of a line (null: none); ff_lines.hip
+constexpr int kLdsStat = 3;
+constexpr int kLdsParts = 14;
+const void* lds_col_kernel(int f32, int mode, int n, int E);
+const void* lds_r2c_kernel(int f32, int in_f32, int odd, int M, int E);
+const void* lds_c2r_kernel(int f32, int out_kind, int odd, int epi, int M, int E);
+template <int PART>
+const void* lds_col_part(int f32, int mode, int n, int E);
+template <int PART>
+const void* lds_r2c_part(int f32, int in_f32, int M, int E);
+template <int PART>
+const void* lds_c2r_part(int f32, int out_kind, int epi, int M, int E);
+
+// Shape of a column kernel of the table: T columns (about 256 threads; at least 64 bytes,
+// at most 256 a row, 512 for short lines; whole 128-byte lines where a one-transform pass
+// has the registers for wider workgroups), the waves per SIMD its registers must allow
+// (one transform takes fewer than the x pass's two), and the split exchange where it lets
+// more workgroups share a CU.
+struct LdsShape {
+  int T, waves, split;
+  int threads, lds;
+};
+__host__ __device__ constexpr LdsShape lds_shape(int n, int E, bool f32, bool x) {
+  LdsShape s{};
+  const int L = n / E, eb = f32 ? 8 : 16;
+  s.T = 4;
+  if (f32 && 8 * L <= max_threads_for(E)) s.T = 8;
+  while (2 * s.T * L <= 256 && 2 * s.T * eb <= (n <= 128 ? 512 : 256)) s.T *= 2;
+  if (!x && E <= 8 && s.T * eb == 64 && 2 * s.T * L <= (f32 ? 1024 : 512)) s.T *= 2;
+  s.threads = s.T * L;
+  if (f32) s.waves = E >= 20 ? 3 : 4;
+  else if (x) s.waves = E >= 16 ? 2 : E > 12 ? 3 : 4;
+  else s.waves = E > 20 ? 2 : E > 12 ? 3 : 4;
+  const int per = (s.threads + 63) / 64, fit = 4 * s.waves / per;
+  const int elems = n * s.T + ((n - 1) >> kColPadShift) + 1, tab = tw_lds_slots(n) * eb;
+  const int whole = (elems * eb + 15) / 16 * 16 + tab, half = (elems * eb / 2 + 15) / 16 * 16 + tab;
+  s.split = 160 * 1024 / whole < fit && 160 * 1024 / whole < 160 * 1024 / half;
+  s.lds = s.split ? half : whole;
+  return s;
+}
 
 template <int E>
 struct PassLaunchers {

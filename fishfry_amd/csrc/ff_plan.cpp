@@ -466,8 +466,53 @@ bool col_cfg_with(int n, int ncols, int elem_bytes, ColCfg& out, int E, int T, i
   out.lds = elems * (size_t)(out.split ? elem_bytes / 2 : elem_bytes);
   // LDS twiddles: the first half of the table after the exchange (16-byte
   // aligned)
-  if (out.stat == 2) out.lds = (out.lds + 15) / 16 * 16 + ne / 2 * (size_t)elem_bytes;
+  if (out.stat == 2) out.lds = (out.lds + 15) / 16 * 16 + (size_t)tw_lds_slots((int)ne) * elem_bytes;
   return out.lds <= 160 * 1024;
+}
+
+// Whether a table's line (n, E) is compiled with the plan lp.
+template <const LdsLine* TABLE, int COUNT, int K = 0>
+static bool lds_line_matches(int n, int E, const LinePlan& lp) {
+  if constexpr (K < COUNT) {
+    constexpr LdsLine c = TABLE[K];
+    if (c.n == n && c.E == E) {
+      constexpr LinePlan s = static_plan<c.n, c.E>();
+      if (s.n != lp.n || s.L != lp.L || s.np != lp.np) return false;
+      for (int p = 0; p < s.np; ++p)
+        if (s.radix[p] != lp.radix[p] || s.ns[p] != lp.ns[p] || s.nsinv[p] != lp.nsinv[p] ||
+            s.twstep[p] != lp.twstep[p])
+          return false;
+      return true;
+    }
+    return lds_line_matches<TABLE, COUNT, K + 1>(n, E, lp);
+  } else {
+    return false;
+  }
+}
+
+void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind) {
+  const int n = c.line.n;
+  if (c.line.bluestein() || c.groups != 1 || c.split || c.stat == 2) return;
+  if (!lds_line_matches<kLdsCols, kNumLdsCols>(n, c.line.E, c.line.lp)) return;
+  const LdsShape s = lds_shape(n, c.line.E, elem_bytes == 8, kind == 2);
+  if (s.T / 2 >= ncols || s.lds > 160 * 1024) return;  // narrow planes
+  c.T = s.T;
+  c.lgT = 0;
+  while ((1 << c.lgT) < c.T) c.lgT++;
+  c.split = s.split;
+  c.stat = kLdsStat;
+  c.lds = s.lds;
+  c.threads = s.threads;
+}
+
+void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes) {
+  if (nz % 2 || c.line.bluestein() || c.stat == 2) return;
+  const int M = nz / 2;
+  if (!c.stat && !lds_line_matches<kLdsRows, kNumLdsRows>(M, c.line.E, c.line.lp)) return;
+  const size_t lds = c.lds + (size_t)tw_lds_slots(M) * elem_bytes;
+  if (lds > 160 * 1024) return;
+  c.lds = lds;
+  c.stat = c.stat ? 2 : kLdsStat;
 }
 
 template <int K>
@@ -517,7 +562,7 @@ bool row_cfg_with(int nz, int elem_bytes, RowCfg& out, int E, int T, int flags) 
     // the first half of the W_M table follows the row tiles in LDS
     if (out.stat != 1 || (flags & FF_TUNE_GENERIC)) return false;
     out.stat = 2;
-    out.lds += (size_t)(M / 2) * elem_bytes;
+    out.lds += (size_t)tw_lds_slots(M) * elem_bytes;
   }
   return out.lds <= 160 * 1024;
 }

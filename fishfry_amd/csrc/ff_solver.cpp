@@ -275,6 +275,19 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     }
   }
 
+  // Lines compiled in with twiddles in LDS, unless tuned
+  for (int prec = 0; prec < nprec; ++prec) {
+    int uE, uT, uF;
+    const int eb = prec ? 8 : 16;
+    const bool pen = p->pencil && prec == mainp;
+    if (!p->fz.n && !tune_lookup(0, n[2] / 2, prec, uE, uT, uF)) row_lds_twiddles(p->zr[prec], n[2], eb);
+    if (!p->fz.n && !tune_lookup(3, n[2] / 2, prec, uE, uT, uF)) row_lds_twiddles(p->zi[prec], n[2], eb);
+    if (!p->fy.n && !tune_lookup(1, n[1], prec, uE, uT, uF))
+      col_lds_twiddles(p->cy[prec], pen ? std::min(p->nh, n[0]) : p->nh, eb, 1);
+    if (!p->fx.n && !p->fy.n && !tune_lookup(2, n[0], prec, uE, uT, uF))
+      col_lds_twiddles(p->cx[prec], pen ? n[1] : p->nh, eb, 2);
+  }
+
   // Planes that fit a CU: their z and y passes as one kernel each way, where the
   // passes would run the same plans in the plain layout.
   for (int prec = 0; prec < nprec; ++prec) {
@@ -990,7 +1003,7 @@ static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, con
   }
   // kernels with LDS twiddles also copy the x axis's finite-difference
   // factors to LDS, after the twiddles
-  const size_t lds = c.lds + (mode == COL_FILTER_FD && c.stat == 2 ? (size_t)c.line.lp.n * sizeof(double) : 0);
+  const size_t lds = c.lds + (mode == COL_FILTER_FD && c.stat >= 2 ? (size_t)c.line.lp.n * sizeof(double) : 0);
   const Launch l{dim3(a.nblocks), dim3(c.threads), lds, s};
   return hip_check(launch_col(c.line.E, prec, mode, c.split, c.groups, c.line.bluestein(), c.stat, l, a),
                    "column pass launch");

@@ -271,7 +271,7 @@ ff_status ff_batch_wait(ff_batch* b, void* stream);
 /* Autotuner: times every valid (elements per thread, lines per workgroup)
  * configuration of each distinct pass of the batch on the given buffers
  * (reps launches each; the buffers' contents are overwritten), records the
- * fastest with ff_tune_set and re-plans.  tuned: passes tuned; ms_before /
+ * fastest with ff_tune_set where it beats the plan's own and re-plans.  tuned: passes tuned; ms_before /
  * ms_after: batch solve time before and after. */
 ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* potential, void* stream, int reps,
                             int* tuned, double* ms_before, double* ms_after);
