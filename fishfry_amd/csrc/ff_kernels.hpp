@@ -606,13 +606,6 @@ __device__ __forceinline__ long long spec_row(const RowArgs& a, long long row) {
 // SN > 0: the plan of the row transform, length SN, is compiled in (even nz).
 // r2c_tile: the work of one workgroup, row block blk (< a.nblocks), with the
 // per-instance fields io (k_r2c: one pass; ff_multi.hip: many instances).
-// Waves per SIMD that the registers of a row kernel must allow: two where many elements
-// per thread would let it take them all.
-template <int E, int SN, bool TWL>
-constexpr int row_waves() {
-  return SN > 0 && TWL && E >= 20 ? 2 : 1;
-}
-
 // TWL (compiled-in plans): the first half of the W_SN table is copied to LDS
 // after the T row tiles and the passes read their twiddles there.
 template <typename F, int SN>
@@ -708,8 +701,15 @@ __device__ __forceinline__ void r2c_tile(const RowArgs& a, const PassInst& io, i
 }
 
 template <typename F, typename IN, int E, bool ODD, bool BL, int SN = 0, bool TWL = false>
-__global__ __launch_bounds__(max_threads_for(E), (row_waves<E, SN, TWL>())) void k_r2c(const RowArgs a) {
+__global__ __launch_bounds__(max_threads_for(E)) void k_r2c(const RowArgs a) {
   r2c_tile<F, IN, E, ODD, BL, SN, TWL>(a, inst_of(a), xcd_remap(blockIdx.x, a.nblocks));
+}
+
+// The kLdsRows kernels: two waves per SIMD where the elements per thread would let them take
+// every register.
+template <typename F, typename IN, int E, int SN>
+__global__ __launch_bounds__(max_threads_for(E), E >= 20 ? 2 : 1) void k_r2c_line(const RowArgs a) {
+  r2c_tile<F, IN, E, false, false, SN, true>(a, inst_of(a), xcd_remap(blockIdx.x, a.nblocks));
 }
 
 // Epilogues of the z inverse: store scale*x, store the residual
@@ -896,8 +896,13 @@ __device__ __forceinline__ void c2r_tile(const RowArgs& a, const PassInst& io, i
 }
 
 template <typename F, typename OUT, int E, bool ODD, int EPI, bool BL, int SN = 0, bool TWL = false>
-__global__ __launch_bounds__(max_threads_for(E), (row_waves<E, SN, TWL>())) void k_c2r(const RowArgs a) {
+__global__ __launch_bounds__(max_threads_for(E)) void k_c2r(const RowArgs a) {
   c2r_tile<F, OUT, E, ODD, EPI, BL, SN, TWL>(a, inst_of(a), xcd_remap(blockIdx.x, a.nblocks));
+}
+
+template <typename F, typename OUT, int E, int EPI, int SN>
+__global__ __launch_bounds__(max_threads_for(E), E >= 20 ? 2 : 1) void k_c2r_line(const RowArgs a) {
+  c2r_tile<F, OUT, E, false, EPI, false, SN, true>(a, inst_of(a), xcd_remap(blockIdx.x, a.nblocks));
 }
 
 // ---------------------------------------------------------------------------

@@ -47,9 +47,9 @@ static const void* r2c_line_of(int f32, int in_f32, int M, int E) {
   if constexpr (K < kNumLdsRows) {
     constexpr LdsLine c = kLdsRows[K];
     if (c.n == M && c.E == E) {
-      if (!f32) return in_f32 ? nullptr : (const void*)&k_r2c<double, double, c.E, false, false, c.n, true>;
-      return in_f32 ? (const void*)&k_r2c<float, float, c.E, false, false, c.n, true>
-                    : (const void*)&k_r2c<float, double, c.E, false, false, c.n, true>;
+      if (!f32) return in_f32 ? nullptr : (const void*)&k_r2c_line<double, double, c.E, c.n>;
+      return in_f32 ? (const void*)&k_r2c_line<float, float, c.E, c.n>
+                    : (const void*)&k_r2c_line<float, double, c.E, c.n>;
     }
     return r2c_line_of<K + kLdsParts>(f32, in_f32, M, E);
   } else {
@@ -62,7 +62,7 @@ static const void* c2r_line_of(int f32, int out_kind, int epi, int M, int E) {
   if constexpr (K < kNumLdsRows) {
     constexpr LdsLine c = kLdsRows[K];
     if (c.n == M && c.E == E) {
-#define FF_C2R(F, OUT, EPI) return (const void*)&k_c2r<F, OUT, c.E, false, EPI, false, c.n, true>
+#define FF_C2R(F, OUT, EPI) return (const void*)&k_c2r_line<F, OUT, c.E, EPI, c.n>
       if (!f32) {
         if (epi == EPI_STORE && out_kind == 0) FF_C2R(double, double, EPI_STORE);
         if (epi == EPI_RESIDUAL && out_kind == 1) FF_C2R(double, float, EPI_RESIDUAL);

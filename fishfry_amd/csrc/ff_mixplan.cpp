@@ -109,7 +109,7 @@ static void build_plan(int n, int prec, std::vector<unsigned char>& buf) {
   memcpy(buf.data(), &mp, sizeof mp);
 }
 
-bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, MixCfg& out) {
+bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, long long lines, MixCfg& out) {
   out = MixCfg{};
   const std::vector<int> rs = mix_radices(n);
   const bool rows = kind == 0 || kind == 3;
@@ -131,6 +131,8 @@ bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, MixCfg& out) {
   while (T > tmin && T * n > 32768 / eb) T /= 2;
   if (dense)
     while (T < 8) T *= 2;
+  // (narrower where the grid would leave CUs without a tile)
+  while (T > std::max(tmin, dense ? 8 : 1) && lines / T < 256) T /= 2;
   while (T > tmin && bytes(T) > 80 * 1024) T /= 2;
   while (T > 1 && bytes(T) > 160 * 1024) T /= 2;
   while (!rows && T > 1 && T / 2 >= ncols) T /= 2;

@@ -493,6 +493,9 @@ static bool lds_line_matches(int n, int E, const LinePlan& lp) {
 void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind) {
   const int n = c.line.n;
   if (c.line.bluestein() || c.groups != 1 || c.split || c.stat == 2) return;
+  // (lines of 160 keep the kernel they have but for the FP64 x pass: 160^3 FP32 68 us
+  // with it, 71 with this; 64x160x128 FP64, y lines, 42 and 44)
+  if (c.stat == 1 && n < 256 && (elem_bytes == 8 || kind == 1)) return;
   if (!lds_line_matches<kLdsCols, kNumLdsCols>(n, c.line.E, c.line.lp)) return;
   const LdsShape s = lds_shape(n, c.line.E, elem_bytes == 8, kind == 2);
   if (s.T / 2 >= ncols || s.lds > 160 * 1024) return;  // narrow planes
@@ -508,6 +511,9 @@ void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind) {
 void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes) {
   if (nz % 2 || c.line.bluestein() || c.stat == 2) return;
   const int M = nz / 2;
+  // (compiled-in rows within a wavefront, which exchange without a workgroup barrier, gain
+  // nothing from it: 128^3 FP64 50.5 us with twiddles from memory, 53.4 from LDS)
+  if (c.stat && 64 % (M / c.line.E) == 0) return;
   if (!c.stat && !lds_line_matches<kLdsRows, kNumLdsRows>(M, c.line.E, c.line.lp)) return;
   const size_t lds = c.lds + (size_t)tw_lds_slots(M) * elem_bytes;
   if (lds > 160 * 1024) return;

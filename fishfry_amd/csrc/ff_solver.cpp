@@ -239,13 +239,17 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
       return m == 1;
     };
     const int M = n[2] % 2 ? n[2] : n[2] / 2;
+    const long long rows = (long long)n[0] * (n[2] % 2 ? (n[1] + 1) / 2 : n[1]);
     // (odd nz: the pairs of a plane are indexed below 2^16)
     if (!p->fz.n && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
-        !(mix_cfg(M, prec, 0, n[1], n[2] % 2, p->mzr[prec]) && mix_cfg(M, prec, 3, n[1], n[2] % 2, p->mzi[prec])))
+        !(mix_cfg(M, prec, 0, n[1], n[2] % 2, rows, p->mzr[prec]) && mix_cfg(M, prec, 3, n[1], n[2] % 2, rows, p->mzi[prec])))
       p->mzr[prec].plan = p->mzi[prec].plan = nullptr;
     const bool pen = p->pencil && prec == mainp;
-    if (!p->fy.n && !smooth(n[1]) && !tuned(1, n[1])) mix_cfg(n[1], prec, 1, pen ? std::max(p->nh, n[0]) : p->nh, false, p->my[prec]);
-    if (!p->fx.n && !p->fy.n && !smooth(n[0]) && !tuned(2, n[0])) mix_cfg(n[0], prec, 2, pen ? n[1] : p->nh, false, p->mx[prec]);
+    const long long yl = (long long)n[0] * p->nh, xl = (long long)n[1] * p->nh;
+    if (!p->fy.n && !smooth(n[1]) && !tuned(1, n[1]))
+      mix_cfg(n[1], prec, 1, pen ? std::max(p->nh, n[0]) : p->nh, false, yl, p->my[prec]);
+    if (!p->fx.n && !p->fy.n && !smooth(n[0]) && !tuned(2, n[0]))
+      mix_cfg(n[0], prec, 2, pen ? n[1] : p->nh, false, xl, p->mx[prec]);
     // one workgroup per tile of a 32-bit grid
     auto fits = [&](MixCfg& c, long long planes, long long lines) {
       if (c.plan && planes * ((lines + c.T - 1) / c.T) > INT_MAX) c.plan = nullptr;
@@ -401,14 +405,16 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
 
 // Whether the plane kernels run a plan's z and y passes, with `instances` solves
 // of it in one launch: always for planes of up to 6144 points, several of which
-// share a CU; larger ones take a CU each, and then need enough of them.  (One
+// share a CU; larger ones take a CU each, and then need enough of them, fewer in the
+// residual of a refinement, whose spectrum stays in place.  (One
 // box, passes and planes: 64^3 FP64 21.3 and 17.8 us; 32x96x32 29 and 17;
-// 1000x64x64 82 and 62; 32x128x128 28 and 38; 256x128x128 74 and 60; FP32
-// 128x128x128 37 and 38, 256x128x128 80 and 60.)
+// 1000x64x64 82 and 62; 32x128x128 28 and 38; 128^3 50 and 53, 256x128x128 74 and 60; FP32
+// 128^3 37 and 38, with a refinement step and planes in its residual 140 and 130,
+// 256x128x128 80 and 60.)
 void plan_choose_planes(ff_plan* p, int instances) {
   const long long planes = (long long)p->n[0] * instances;
   for (int prec = 0; prec < 2; ++prec)
-    p->plane[prec] = p->planes_fit[prec] && ((long long)p->n[1] * p->n[2] <= 6144 || planes >= (prec ? 192 : 128));
+    p->plane[prec] = p->planes_fit[prec] && ((long long)p->n[1] * p->n[2] <= 6144 || planes >= (!prec && p->opt.precision != FF_FP64 ? 128 : 192));
 }
 
 static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
