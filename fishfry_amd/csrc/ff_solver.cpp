@@ -240,8 +240,10 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     };
     const int M = n[2] % 2 ? n[2] : n[2] / 2;
     const long long rows = (long long)n[0] * (n[2] % 2 ? (n[1] + 1) / 2 : n[1]);
-    // (odd nz: the pairs of a plane are indexed below 2^16)
-    if (!p->fz.n && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
+    // (odd nz: the pairs of a plane are indexed below 2^16.  Small grids whose odd nz is
+    // smooth with few elements per thread stay: 30x25x27, rows 4.4 us and here 6)
+    const bool few = n[2] % 2 && smooth(n[2]) && p->zr[prec].line.E <= 6 && p->N < (1LL << 20);
+    if (!p->fz.n && !few && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
         !(mix_cfg(M, prec, 0, n[1], n[2] % 2, rows, p->mzr[prec]) && mix_cfg(M, prec, 3, n[1], n[2] % 2, rows, p->mzi[prec])))
       p->mzr[prec].plan = p->mzi[prec].plan = nullptr;
     const bool pen = p->pencil && prec == mainp;
