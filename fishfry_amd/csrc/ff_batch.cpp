@@ -225,7 +225,7 @@ bool groups_current(const ff_batch* b, double* const* d, double* const* p) {
 // ---- FF_BATCH_STEPS -----------------------------------------------------------
 
 // The multi-shape descriptor of a recorded column pass, or false when no
-// multi-shape variant runs it (Bluestein lines, tuning variants, blocked
+// multi-shape variant runs it (Bluestein and mixed-radix lines, tuning variants, blocked
 // layouts, lengths without a compiled-in variant).  The descriptor keeps the
 // recorded arguments and takes the variant's tile width; lds: the variant's
 // LDS bytes.

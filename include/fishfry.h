@@ -207,7 +207,9 @@ typedef struct ff_tune {
 
 ff_status ff_tune_set(const ff_tune* t);
 void ff_tune_reset(void);
-/* The configuration a plan created now would use for (kind, n, precision);
+/* The configuration a plan created now would use for (kind, n, precision)
+ * (an untuned plan may run the same elements per thread with the plan compiled
+ * in and the twiddles in LDS, which gives the same results);
  * ncols is the column count of the pass (nh), used to cap T. */
 ff_status ff_tune_query(int kind, int n, int precision, int ncols, ff_tune* out);
 ff_status ff_solve_pass(const ff_plan* plan, int pass, const double* src, double* dst, void* stream);
