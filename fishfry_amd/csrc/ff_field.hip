@@ -327,6 +327,17 @@ static FieldTiles field_tiling(const FieldArgs& a) {
   return t;
 }
 
+// A kernel over the tiles with the dynamic LDS of their factors: 76 KB at 64
+// planes and 32 modes.  Above 64 KB a kernel has to be given it first.
+static hipError_t field_launch(const void* fn, unsigned grid, const FieldTiles& t, void** argv, hipStream_t s) {
+  const size_t lds = t.doubles() * sizeof(double);
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  return hipLaunchKernel(fn, dim3(grid), dim3(kFieldThreads), argv, lds, s);
+}
+
 ff_status field_check(const ff_field* f) {
   if (!f) return set_error(FF_ERR_INVALID, "ff_field: null descriptor");
   for (int c = 0; c < 3; ++c)
@@ -344,13 +355,10 @@ ff_status field_init(const ff_field* f, double* out, hipStream_t s) {
   field_args(*f, a);
   const FieldTiles t = field_tiling(a);
   const unsigned grid = (unsigned)std::min<long long>(t.tiles, 1 << 20);
-  const size_t lds = t.doubles() * sizeof(double);
-  switch (field_m4(a)) {
-    case 0: hipLaunchKernelGGL(k_field_init<0>, dim3(grid), dim3(kFieldThreads), lds, s, a, t, out); break;
-    case 4: hipLaunchKernelGGL(k_field_init<4>, dim3(grid), dim3(kFieldThreads), lds, s, a, t, out); break;
-    default: hipLaunchKernelGGL(k_field_init<8>, dim3(grid), dim3(kFieldThreads), lds, s, a, t, out); break;
-  }
-  return hip_check(hipGetLastError(), "k_field_init launch");
+  const void* const fns[3] = {(const void*)&k_field_init<0>, (const void*)&k_field_init<4>,
+                              (const void*)&k_field_init<8>};
+  void* argv[] = {&a, const_cast<FieldTiles*>(&t), &out};
+  return hip_check(field_launch(fns[field_m4(a) / 4], grid, t, argv, s), "k_field_init launch");
 }
 
 static_assert(kDiffDoubles == 3 * DIFF_BLOCKS + 3 && kDiffResult == 3 * DIFF_BLOCKS, "diff work area");
@@ -375,13 +383,10 @@ ff_status field_diff_enqueue(const ff_field* f, const double* phi, double* parti
   field_args(*f, a);
   const FieldTiles t = field_tiling(a);
   const int nb = (int)std::min<long long>(t.tiles, DIFF_BLOCKS);
-  const size_t lds = t.doubles() * sizeof(double);
-  switch (field_m4(a)) {
-    case 0: hipLaunchKernelGGL(k_field_diff<0>, dim3(nb), dim3(DIFF_THREADS), lds, s, a, t, phi, partial); break;
-    case 4: hipLaunchKernelGGL(k_field_diff<4>, dim3(nb), dim3(DIFF_THREADS), lds, s, a, t, phi, partial); break;
-    default: hipLaunchKernelGGL(k_field_diff<8>, dim3(nb), dim3(DIFF_THREADS), lds, s, a, t, phi, partial); break;
-  }
-  st = hip_check(hipGetLastError(), "k_field_diff launch");
+  const void* const fns[3] = {(const void*)&k_field_diff<0>, (const void*)&k_field_diff<4>,
+                              (const void*)&k_field_diff<8>};
+  void* argv[] = {&a, const_cast<FieldTiles*>(&t), &phi, &partial};
+  st = hip_check(field_launch(fns[field_m4(a) / 4], (unsigned)nb, t, argv, s), "k_field_diff launch");
   if (st != FF_OK) return st;
   hipLaunchKernelGGL(k_field_diff_final, dim3(1), dim3(DIFF_THREADS), 0, s, partial, nb, partial + 3 * DIFF_BLOCKS);
   return hip_check(hipGetLastError(), "k_field_diff_final launch");
