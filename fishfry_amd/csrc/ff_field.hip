@@ -318,11 +318,12 @@ static int field_m4(const FieldArgs& a) { return a.nmodes == 0 ? 0 : (a.nmodes <
 // chip; at least 4, one per wave.
 static FieldTiles field_tiling(const FieldArgs& a) {
   FieldTiles t;
-  t.tj = (a.nj + kRows - 1) / kRows;
-  t.tk = (a.nk + kCols - 1) / kCols;
+  // (extents up to 2^31 - 1: no sum with a tile's width)
+  t.tj = 1 + (a.nj - 1) / kRows;
+  t.tk = 1 + (a.nk - 1) / kCols;
   const long long across = (long long)t.tj * t.tk;
   t.planes = (int)std::max<long long>(4, std::min<long long>(kMaxPlanes, a.ni * across / kFieldGroups));
-  t.tiles = across * ((a.ni + t.planes - 1) / t.planes);
+  t.tiles = across * (1 + (a.ni - 1) / t.planes);
   t.modes4 = 4 * field_m4(a);
   return t;
 }

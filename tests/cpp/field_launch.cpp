@@ -139,6 +139,13 @@ int main() {
       check(n, n, n, nmodes);
       check(n, 1, 3 * n, nmodes);
     }
+  // extents up to the type's largest
+  const int top = 2147483647;
+  for (int n : {top, top - 1, top - 15, top - 16, top - 62, top - 63, top - 255, top - 256}) {
+    check(n, 1, 1, 17);
+    check(1, n, 1, 17);
+    check(1, 1, n, 17);
+  }
   std::printf("field launches ok\n");
   return 0;
 }

@@ -2,7 +2,7 @@
 the host code runs under AddressSanitizer and UndefinedBehaviorSanitizer with the
 HIP launch calls replaced by stand-ins (tests/cpp/field_launch.cpp) that refuse
 dynamic LDS above 64 KB unless the kernel has been given it, and grids without
-workgroups, for grids of every planes-per-tile."""
+workgroups, for grids of every planes-per-tile and extents up to 2^31 - 1."""
 import os
 import subprocess
 
