@@ -37,24 +37,25 @@ uint32_t magic(int v) { return v > 1 ? (uint32_t)(((1ull << 32) + (uint64_t)v - 
 }  // namespace
 
 std::vector<int> mix_radices(int n) {
+  if (n < 2) return {};
+  // factors up to 13 are butterflies; what is left once they are out has only prime
+  // factors from 17 on, which trial division finds in ascending order
   std::vector<int> dense, small;
-  int m = n;
-  for (int p = 17; (long long)p * p <= m; p += 2) {
-    while (m % p == 0) {
-      dense.push_back(p);
-      m /= p;
+  int m = 1, rest = n;
+  for (int p : {2, 3, 5, 7, 11, 13}) {
+    while (rest % p == 0) {
+      rest /= p;
+      m *= p;
     }
   }
-  // what is left: factors up to 13, times at most one prime above
-  int rest = m;
-  for (int p : {2, 3, 5, 7, 11, 13})
-    while (rest % p == 0) rest /= p;
-  if (rest > 1) {
-    dense.push_back(rest);
-    m /= rest;
+  for (int p = 17; (long long)p * p <= rest; p += 2) {
+    while (rest % p == 0) {
+      dense.push_back(p);
+      rest /= p;
+    }
   }
-  std::sort(dense.begin(), dense.end());
-  if (n < 2 || (!dense.empty() && dense.back() > kMixMaxDense)) return {};
+  if (rest > 1) dense.push_back(rest);
+  if (!dense.empty() && dense.back() > kMixMaxDense) return {};
   fewest_stages(m, small);
   std::sort(small.begin(), small.end(), [](int a, int b) { return a > b; });
   small.insert(small.end(), dense.begin(), dense.end());
