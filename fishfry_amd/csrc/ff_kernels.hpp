@@ -125,6 +125,7 @@ struct ColArgs {
   // spectral filter); the axis term is g[k] * dd
   const double *symx, *symy, *symz;
   double* dc_out;  // FILTER / SYMBOL: receives the forward (0,0,0) term (sum of the input)
+  int dc_add;      // it is added to what dc_out holds (FP32 passes: the sum a correction's residual still has)
   const void* tw;
   LinePlan lp;
   int nline;                     // transform length (lp.n: engine length; larger for Bluestein)
@@ -267,7 +268,11 @@ __device__ __forceinline__ void col_line(cx<F> (&v)[E], const ColArgs& a, const 
     }
     const bool jv = a.cols_j ? valid : true, kv = a.cols_j ? true : valid;  // index in range
     // the (0,0,0) term before the multiply is the sum of the input field
-    if (io.dc_out && valid && r0 == 0 && plo == 0 && jj == 0 && kk == 0) *glb<double>(io.dc_out) = double(v[0].x);
+    if (io.dc_out && valid && r0 == 0 && plo == 0 && jj == 0 && kk == 0) {
+      FF_GLB double* dc = glb<double>(io.dc_out);
+      if constexpr (std::is_same<F, float>::value) *dc = a.dc_add ? *dc + double(v[0].x) : double(v[0].x);
+      else *dc = v[0].x;
+    }
     if constexpr (MODE == COL_FILTER_FD) {
       // columns outside the plane and Bluestein positions past the line read
       // entry 0 (their values are never stored)

@@ -13,6 +13,8 @@
 // row segments of 64 bytes and more.  Two buffers in turn cost one barrier per
 // stage instead of two, and let a stage's butterflies be spread over all
 // threads whatever its radix.
+#include <type_traits>
+
 #include "ff_mixed.hpp"
 
 #ifndef FF_MIX_PART
@@ -546,6 +548,7 @@ struct FilterSnk {
   double ddi, ddj, ddk;
   const FF_GLB double *symx, *symy, *symz;
   FF_GLB double* dc;
+  int dc_add;
   struct Line {
     cx<F>* p;
     int lg, jk, nx;       // jk: j | kh
@@ -553,6 +556,7 @@ struct FilterSnk {
     double ddk;
     const FF_GLB double* symx;
     FF_GLB double* dc;
+    int dc_add;
     __device__ __forceinline__ F factor(int ii) const {
       if constexpr (MODE == COL_FILTER_FD) {
         const double s2 = fmadd(dk, ddk, fmadd(symx[ii], ddi, dj));
@@ -564,15 +568,16 @@ struct FilterSnk {
         else return F(-s2);
       }
     }
-    // (the (0,0,0) term before the multiply is the sum of the input field)
+    // the (0,0,0) term before the multiply is the sum of the input field
+    __device__ __forceinline__ void put_dc(F v) const { *dc = std::is_same<F, float>::value && dc_add ? *dc + double(v) : double(v); }
     __device__ __forceinline__ void operator()(int pos, cx<F> v) const {
       const F d = factor(pos);
-      if (dc && !(pos | jk)) *dc = double(v.x);
+      if (dc && !(pos | jk)) put_dc(v.x);
       p[pos << lg] = cx<F>{d * v.x, d * v.y};
     }
     __device__ __forceinline__ void operator()(int pos, int part, F v) const {
       const F d = factor(pos);
-      if (dc && !(pos | jk | part)) *dc = double(v);
+      if (dc && !(pos | jk | part)) put_dc(v);
       reinterpret_cast<F*>(p + (pos << lg))[part] = d * v;
     }
   };
@@ -588,6 +593,7 @@ struct FilterSnk {
     l.ddi = ddi;
     l.ddk = ddk;
     l.dc = dc;
+    l.dc_add = dc_add;
     l.symx = symx;
     if constexpr (MODE == COL_FILTER_FD) {
       l.dj = symy[jj] * ddj;
@@ -630,7 +636,7 @@ __global__ __launch_bounds__(kMixThreads) void k_mix_col(const ColArgs a) {
       const FilterSnk<F, MODE> filter{mix_tile<F, false>(lds, last ^ 1, stride, a.T, a.lgT, 0, tab),
                                       outer, col0, a.ncols, a.cols_j, a.nx, a.ny, io.ddi, io.ddj, io.ddk,
                                       glb<const double>(a.symx), glb<const double>(a.symy),
-                                      glb<const double>(a.symz), glb<double>(io.dc_out)};
+                                      glb<const double>(a.symz), glb<double>(io.dc_out), a.dc_add};
       mix_stages<-1, F, false>(mp, p, lds, b, stride, a.T, a.lgT, 0, tw, tab, filter);
       __syncthreads();
       b = last ^ 1;

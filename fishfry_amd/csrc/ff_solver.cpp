@@ -894,7 +894,7 @@ struct SubLines {
 // Bluestein tables bl); sub: four-step geometry (null: whole lines); mix: the
 // mixed-radix tile that runs it instead (null: none).
 static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, const void* src, void* dst,
-                             hipStream_t s, double* dc_out, int lay_in, int lay_out, int outer0, int nouter,
+                             hipStream_t s, DcOut dc_out, int lay_in, int lay_out, int outer0, int nouter,
                              const ColCfg& c, const void* tw, const void* const* bl, const SubLines* sub,
                              const MixCfg* mix = nullptr) {
   if (src == dst && lay_in != lay_out) return set_error(FF_ERR_INVALID, "in-place column pass must keep its layout");
@@ -991,7 +991,8 @@ static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, con
     a.ddj = p->ddj;
     a.ddk = p->ddk;
   }
-  a.dc_out = dc_out;
+  a.dc_out = dc_out.p;
+  a.dc_add = dc_out.add;
   a.tw = tw;
   a.lp = c.line.lp;
   a.nline = c.line.n;
@@ -1028,7 +1029,7 @@ static ff_status run_col_cfg(const ff_plan* p, int prec, int axis, int mode, con
 // order (jmap); an x pass of four-step lines runs A, B with the filter at
 // frequency i = k2 + n2*k1, then A^-1.
 ff_status run_col(const ff_plan* p, int prec, int axis, int mode, const void* src, void* dst, hipStream_t s,
-                  double* dc_out, int lay_in, int lay_out, int outer0, int nouter) {
+                  DcOut dc_out, int lay_in, int lay_out, int outer0, int nouter) {
   const ff_plan::FourStep& fs = axis == 1 ? p->fy : p->fx;
   if (!fs.n) {
     const ColCfg& c = axis == 1 ? p->cy[prec] : p->cx[prec];
@@ -1052,7 +1053,7 @@ ff_status run_col(const ff_plan* p, int prec, int axis, int mode, const void* sr
     return run_col_cfg(p, prec, axis, m, in, out, s, nullptr, LAY_PLAIN, LAY_PLAIN, 0, -1, fs.c2[prec], fs.tw2[prec],
                        fs.bl2[prec], &ga);
   };
-  auto B = [&](int m, const void* in, void* out, double* dc) {
+  auto B = [&](int m, const void* in, void* out, DcOut dc) {
     return run_col_cfg(p, prec, axis, m, in, out, s, dc, LAY_PLAIN, LAY_PLAIN, 0, -1, fs.c1[prec], fs.tw1[prec],
                        fs.bl1[prec], &gb);
   };
@@ -1075,7 +1076,7 @@ ff_status run_col(const ff_plan* p, int prec, int axis, int mode, const void* sr
 // src (FP64 f or the FP32 residual r) to phi (stored or accumulated): in
 // place in the work area (plain layout), or, with the pencil layout, between
 // its two halves (each holds one FP32 spectrum).
-static ff_status fp32_round_trip(const ff_plan* p, int in_f32, const void* src, double* phi, int epi, double* dc_col,
+static ff_status fp32_round_trip(const ff_plan* p, int in_f32, const void* src, double* phi, int epi, DcOut dc_col,
                                  const double* shiftp, hipStream_t s) {
   void* a = p->spec;
   void* b = p->pencil ? static_cast<void*>(static_cast<char*>(p->spec) + p->Nh * 8) : p->spec;
@@ -1129,8 +1130,13 @@ static ff_status solve_fp32_refine(const ff_plan* p, const double* f, double* ph
       }
       if (st) return st;
     }
-    // correction in FP32: phi += L_h^-1 r - mean(phi)
-    if ((st = fp32_round_trip(p, 1, p->res, phi, EPI_ACCUM, nullptr, p->dc, s))) return st;
+    // correction in FP32: phi += L_h^-1 r - mean(phi).  sum(f) is the FP32
+    // passes' own and off by their rounding, so r keeps a constant, 1e-9 of f
+    // beside a second residual of 1e-13, which its FP32 passes leak into the low modes; r's
+    // sum, added to it, takes the constant out of the next residual
+    // (131x6x10, f + 1, two steps: worst of six 1.1e-13, now as without the 1)
+    const DcOut sum_r = it + 1 < p->opt.refine_steps ? DcOut(p->dcf, 1) : DcOut();
+    if ((st = fp32_round_trip(p, 1, p->res, phi, EPI_ACCUM, sum_r, p->dc, s))) return st;
   }
   return FF_OK;
 }

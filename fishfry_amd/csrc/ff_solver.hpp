@@ -90,8 +90,15 @@ ff_status run_zfwd(const ff_plan* p, int prec, int in_f32, const void* src, void
 // spectrum layouts: plain [i][j][kh]; blocked y [kb][i][j][kt] and x
 // [kb][j][i][kt]; pencil A [i][kh][j], B [kh][j][i] and D [kh][i][j]
 enum { LAY_PLAIN = 0, LAY_Y = 1, LAY_X = 2, LAY_A = 3, LAY_B = 4, LAY_D = 5 };
+// Where the x pass leaves the sum of its input (null: nowhere); add (FP32 passes):
+// added to what is there.
+struct DcOut {
+  double* p;
+  int add;
+  DcOut(double* to = nullptr, int a = 0) : p(to), add(a) {}
+};
 ff_status run_col(const ff_plan* p, int prec, int axis, int mode, const void* src, void* dst, hipStream_t s,
-                  double* dc_out = nullptr, int lay_in = LAY_PLAIN, int lay_out = LAY_PLAIN, int outer0 = 0,
+                  DcOut dc_out = nullptr, int lay_in = LAY_PLAIN, int lay_out = LAY_PLAIN, int outer0 = 0,
                   int nouter = -1);
 ff_status run_zinv(const ff_plan* p, int prec, int out_kind, int epi, const void* src, void* dst, const double* f,
                    const double* shiftp, hipStream_t s, int lay_in = LAY_PLAIN, long long row0 = 0,
