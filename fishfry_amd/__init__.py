@@ -249,6 +249,18 @@ def _stream(stream) -> int:
     return int(stream.cuda_stream)
 
 
+def _described(fn, handle, what: str) -> str:
+    """The JSON description that fn writes, in a buffer that grows until it holds it."""
+    size = 4096
+    while True:
+        buf = ctypes.create_string_buffer(size)
+        status = fn(handle, buf, size)
+        if status == 0 or "too small" not in last_error():
+            check(status, what)
+            return buf.value.decode()
+        size *= 2
+
+
 def reference_bytes(n: Sequence[int], m: Sequence[int] = (1, 1, 1)) -> int:
     """The reference's per-array byte formula (ParisPencil.cpp:49-75)."""
     return int(lib().ff_reference_bytes(_i3(n), _i3(m)))
@@ -319,9 +331,7 @@ class ParisPencil:
         check(lib().ff_solve_pass(self._h, p, _ptr(src), _ptr(dst), _stream(stream)), f"pass {p}")
 
     def describe(self) -> str:
-        buf = ctypes.create_string_buffer(4096)
-        check(lib().ff_plan_describe(self._h, buf, len(buf)), "describe")
-        return buf.value.decode()
+        return _described(lib().ff_plan_describe, self._h, "describe")
 
     def close(self) -> None:
         if getattr(self, "_h", None) is not None and self._h.value:
@@ -404,9 +414,7 @@ class Batch:
         return t.value, b.value, a.value
 
     def describe(self) -> str:
-        buf = ctypes.create_string_buffer(1024 * (self.count + 4))
-        check(lib().ff_batch_describe(self._h, buf, len(buf)), "batch describe")
-        return buf.value.decode()
+        return _described(lib().ff_batch_describe, self._h, "batch describe")
 
     def close(self) -> None:
         if getattr(self, "_h", None) is not None and self._h.value:

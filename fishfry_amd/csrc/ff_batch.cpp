@@ -3,6 +3,7 @@
 // through the multi-shape kernels (ff_multi.hpp), optionally captured in a
 // HIP graph, and the autotuner.
 #include <algorithm>
+#include <array>
 #include <climits>
 #include <cmath>
 #include <cstdint>
@@ -53,6 +54,7 @@ using namespace ff;
 struct BatchGroup {
   std::vector<int> inst;         // instances, in batch order
   std::vector<PassLaunch> ops;   // the group's launches (per-instance fields from the table)
+  int plane[2] = {0, 0};         // z and y passes as plane kernels (FP64, FP32)
 };
 
 struct StepLaunch {
@@ -139,6 +141,7 @@ ff_status prepare_groups(ff_batch* b, double* const* d, double* const* p) {
   b->groups_ok = false;  // the old groups' table may be freed below
   b->groups.clear();
   std::vector<std::vector<PassLaunch>> rec(b->count);
+  std::vector<std::array<int, 2>> planes(b->count);
   for (int i = 0; i < b->count; ++i) {
     if (solo(b, i)) continue;
     // (the group's instances fill the chip together)
@@ -148,6 +151,7 @@ ff_status prepare_groups(ff_batch* b, double* const* d, double* const* p) {
               b->items[k].precision == b->items[i].precision && b->items[k].refine_steps == b->items[i].refine_steps;
     ff_plan plan = *b->plans[i];
     plan_choose_planes(&plan, same);
+    planes[i] = {plan.plane[0], plan.plane[1]};
     set_launch_recorder(&rec[i]);
     const ff_status st = solve_enqueue(&plan, d[i], p[i], nullptr, nullptr);
     set_launch_recorder(nullptr);
@@ -174,6 +178,7 @@ ff_status prepare_groups(ff_batch* b, double* const* d, double* const* p) {
     if (!home) {
       groups.emplace_back();
       home = &groups.back();
+      std::copy(planes[i].begin(), planes[i].end(), home->plane);
     }
     home->inst.push_back(i);
   }
@@ -781,7 +786,7 @@ ff_status ff_batch_describe(const ff_batch* b, char* buf, size_t len) {
      << ",\"graph\":" << (b->exec ? 1 : 0) << ",\"groups\":[";
   for (size_t g = 0; g < b->groups.size(); ++g) {
     os << (g ? "," : "") << "{\"instances\":" << b->groups[g].inst.size() << ",\"launches\":" << b->groups[g].ops.size()
-       << "}";
+       << ",\"planes\":[" << b->groups[g].plane[0] << "," << b->groups[g].plane[1] << "]}";
   }
   os << "],\"steps\":[";
   for (size_t f = 0; f < b->fams.size(); ++f) {

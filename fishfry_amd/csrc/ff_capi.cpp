@@ -204,22 +204,27 @@ ff_status ff_plan_describe(const ff_plan* p, char* buf, size_t len) {
   };
   s += axis("y", p->fy, p->cy[0]) + ",";
   s += axis("x", p->fx, p->cx[0]);
-  // passes run by the mixed-radix kernels: line length, lines per workgroup and radices
-  const MixCfg* mix[4] = {&p->mzr[0], &p->mzi[0], &p->my[0], &p->mx[0]};
+  // passes run by the mixed-radix kernels, FP64 and FP32: line length, lines per workgroup and radices
   static const char* mixkey[4] = {"z", "zi", "y", "x"};
-  s += ",\"mixed\":{";
-  bool first = true;
-  for (int k = 0; k < 4; ++k) {
-    if (!mix[k]->plan) continue;
-    snprintf(tmp, sizeof tmp, "%s\"%s\":{\"n\":%d,\"T\":%d,\"lds\":%zu,\"radices\":[", first ? "" : ",", mixkey[k],
-             mix[k]->n, mix[k]->T, mix[k]->lds);
-    s += tmp;
-    const std::vector<int> rs = mix_radices(mix[k]->n);
-    for (size_t i = 0; i < rs.size(); ++i) s += (i ? "," : "") + std::to_string(rs[i]);
-    s += "]}";
-    first = false;
+  for (int prec = 0; prec < 2; ++prec) {
+    const MixCfg* mix[4] = {&p->mzr[prec], &p->mzi[prec], &p->my[prec], &p->mx[prec]};
+    s += prec ? ",\"mixed_fp32\":{" : ",\"mixed\":{";
+    bool first = true;
+    for (int k = 0; k < 4; ++k) {
+      if (!mix[k]->plan) continue;
+      snprintf(tmp, sizeof tmp, "%s\"%s\":{\"n\":%d,\"T\":%d,\"lds\":%zu,\"radices\":[", first ? "" : ",", mixkey[k],
+               mix[k]->n, mix[k]->T, mix[k]->lds);
+      s += tmp;
+      const std::vector<int> rs = mix_radices(mix[k]->n);
+      for (size_t i = 0; i < rs.size(); ++i) s += (i ? "," : "") + std::to_string(rs[i]);
+      s += "]}";
+      first = false;
+    }
+    s += "}";
   }
-  s += "}";
+  // z and y passes run as plane kernels, FP64 and FP32
+  snprintf(tmp, sizeof tmp, ",\"planes\":[%d,%d]", p->plane[0], p->plane[1]);
+  s += tmp;
   s += "}";
   if (s.size() + 1 > len) return set_error(FF_ERR_INVALID, "ff_plan_describe: buffer too small");
   memcpy(buf, s.c_str(), s.size() + 1);

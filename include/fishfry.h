@@ -156,7 +156,11 @@ const char* ff_last_error(void);
  * (ParisPencil.cpp:24-26,49-75), without creating a plan. */
 size_t ff_reference_bytes(const int n[3], const int m[3]);
 
-/* Human-readable JSON description of a plan (radix plans, tiles, bytes). */
+/* Human-readable JSON description of a plan (radix plans, tiles, bytes), of up
+ * to about 2 KB: "z", "zi", "y" and "x" are the register engine's FP64
+ * configurations; passes listed in "mixed" (FP64) or "mixed_fp32" run the
+ * mixed-radix kernels instead, and z and y passes run as plane kernels where
+ * "planes" (FP64, FP32) says so. */
 ff_status ff_plan_describe(const ff_plan* plan, char* buf, size_t len);
 
 /* One pass of the solve, for per-pass parity checks and timing:
@@ -207,9 +211,11 @@ typedef struct ff_tune {
 
 ff_status ff_tune_set(const ff_tune* t);
 void ff_tune_reset(void);
-/* The configuration a plan created now would use for (kind, n, precision)
- * (an untuned plan may run the same elements per thread with the plan compiled
- * in and the twiddles in LDS, which gives the same results);
+/* The register engine's configuration of (kind, n, precision), which a plan
+ * created now would use where it runs that engine.  An untuned plan may run the
+ * same elements per thread with the plan compiled in and the twiddles in LDS
+ * or in a plane kernel (the same results), and lengths with a prime factor above 5 and odd
+ * rows in mixed-radix kernels (other rounding): ff_plan_describe says which.
  * ncols is the column count of the pass (nh), used to cap T. */
 ff_status ff_tune_query(int kind, int n, int precision, int ncols, ff_tune* out);
 ff_status ff_solve_pass(const ff_plan* plan, int pass, const double* src, double* dst, void* stream);

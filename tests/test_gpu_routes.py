@@ -1,0 +1,87 @@
+"""Which kernels a plan takes, as its description reports them: plane kernels for
+the shapes and mixed radices for the lengths that test_gpu_plane.py and
+test_gpu_mixed.py compare, so that those comparisons are with another kernel; none of
+them under the overrides that those tests use, nor where a rule excludes them."""
+import json
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import fishfry_amd as ff  # noqa: E402
+from test_gpu_mixed import LENGTHS  # noqa: E402
+from test_gpu_plane import SHAPES  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def described(n, **kw):
+    lo, hi, _ = ff.benchmark_grid(n)
+    with ff.ParisPencil(n, lo, hi, **kw) as p:
+        return json.loads(p.describe())
+
+
+REFINED = dict(precision=ff.FF_FP32_REFINE, refine_steps=2)
+
+
+@pytest.mark.parametrize("n", SHAPES)
+def test_planes(n):
+    assert described(n)["planes"] == [1, 0]
+    assert described(n, **REFINED)["planes"] == [1, 1]
+    for flags in (ff.FF_PENCIL_LAYOUT, ff.FF_BLOCKED_LAYOUT):
+        assert described(n, flags=flags)["planes"] == [0, 0]
+    try:
+        for p in (0, 1):
+            t = ff.tune_query(0, n[2] // 2, p, 1)
+            ff.tune_set(0, n[2] // 2, p, t.E, t.T, 0)
+        assert described(n)["planes"] == [0, 0]
+        assert described(n, **REFINED)["planes"] == [0, 0]
+    finally:
+        ff.tune_reset()
+
+
+def largest_prime(n):
+    p, top = 2, 1
+    while n > 1:
+        while n % p == 0:
+            n //= p
+            top = p
+        p += 1
+    return top
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_mixed(n):
+    top = largest_prime(n)
+    for prec, key, limit, pairs in ((0, "mixed", 200, 300), (1, "mixed_fp32", 300, 420)):
+        kw = REFINED if prec else {}
+        for g, axes, most in (((n, 6, 10), ["x"], limit), ((5, n, 8), ["y"], limit), ((3, 4, 2 * n), ["z", "zi"], limit),
+                              ((4, 5, n), ["z", "zi"], pairs)):
+            if g[2] == n and n % 2 == 0:
+                continue
+            got = described(g, **kw)[key]
+            assert sorted(a for a in got if got[a]["n"] == n) == (sorted(axes) if top <= most else []), (g, key)
+        # a plain FP32 solve stays on the register engine
+        assert described((5, n, 8), precision=ff.FF_FP32_REFINE)["mixed_fp32"] == {}
+        try:
+            t = ff.tune_query(1, n, prec, 5)
+            ff.tune_set(1, n, prec, t.E, t.T, 0)
+            assert "y" not in described((5, n, 8), **kw)[key]
+        finally:
+            ff.tune_reset()
+
+
+def test_groups_and_long_descriptions():
+    """Planes that a group fills the chip with, and a batch whose plans' descriptions are long."""
+    b = ff.Batch([dict(n=(40, 128, 128))] * 5, flags=ff.FF_BATCH_GROUPED)
+    d = [torch.zeros(b.bytes(i) // 8, dtype=torch.float64, device="cuda") for i in range(5)]
+    p = [torch.zeros_like(x) for x in d]
+    b.solve(d, p)
+    b.wait()
+    got = json.loads(b.describe())
+    assert [g["planes"] for g in got["groups"]] == [[1, 0]] and got["plans"][0]["planes"] == [0, 0]
+    b.close()
+    shapes = [(1001, 924, 819 + 2 * k) for k in range(48)]
+    b = ff.Batch([dict(n=n) for n in shapes])
+    assert [tuple(q["n"]) for q in json.loads(b.describe())["plans"]] == shapes
+    b.close()
