@@ -135,6 +135,23 @@ ff_status make_plans(ff_batch* b) {
   return FF_OK;
 }
 
+// The plan of instance i with the z and y passes that the batch's mode runs: a
+// group's instances fill the chip with planes together, and the step mode runs the
+// passes one by one (plane kernels have no multi-shape variant).
+ff_plan mode_plan(const ff_batch* b, int i) {
+  ff_plan plan = *b->plans[i];
+  if (b->flags & FF_BATCH_GROUPED) {
+    int same = 0;
+    for (int k = 0; k < b->count; ++k)
+      same += std::equal(b->items[k].n, b->items[k].n + 3, b->items[i].n) &&
+              b->items[k].precision == b->items[i].precision && b->items[k].refine_steps == b->items[i].refine_steps;
+    plan_choose_planes(&plan, same);
+  } else if (b->flags & FF_BATCH_STEPS) {
+    plan.plane[0] = plan.plane[1] = 0;
+  }
+  return plan;
+}
+
 // Records one solve per instance, forms the groups and uploads their
 // per-instance tables (blocking: waits for the device before rewriting them).
 ff_status prepare_groups(ff_batch* b, double* const* d, double* const* p) {
@@ -144,13 +161,7 @@ ff_status prepare_groups(ff_batch* b, double* const* d, double* const* p) {
   std::vector<std::array<int, 2>> planes(b->count);
   for (int i = 0; i < b->count; ++i) {
     if (solo(b, i)) continue;
-    // (the group's instances fill the chip together)
-    int same = 0;
-    for (int k = 0; k < b->count; ++k)
-      same += std::equal(b->items[k].n, b->items[k].n + 3, b->items[i].n) &&
-              b->items[k].precision == b->items[i].precision && b->items[k].refine_steps == b->items[i].refine_steps;
-    ff_plan plan = *b->plans[i];
-    plan_choose_planes(&plan, same);
+    const ff_plan plan = mode_plan(b, i);
     planes[i] = {plan.plane[0], plan.plane[1]};
     set_launch_recorder(&rec[i]);
     const ff_status st = solve_enqueue(&plan, d[i], p[i], nullptr, nullptr);
@@ -317,8 +328,7 @@ ff_status prepare_steps(ff_batch* b, double* const* d, double* const* p) {
   for (int i = 0; i < b->count; ++i) {
     if (solo(b, i)) continue;
     set_launch_recorder(&rec[i]);
-    ff_plan plan = *b->plans[i];  // the passes one by one: plane kernels have no multi-shape variant
-    plan.plane[0] = plan.plane[1] = 0;
+    const ff_plan plan = mode_plan(b, i);
     const ff_status st = solve_enqueue(&plan, d[i], p[i], nullptr, nullptr);
     set_launch_recorder(nullptr);
     if (st != FF_OK) return st;
@@ -666,13 +676,16 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
   if (st == FF_OK) st = hip_check(hipEventCreate(&e1), "event");
   auto time_batch = [&](double* out) {
     ff_status r = enqueue_all(b, density, potential, s);  // warm up
-    if (r == FF_OK) r = hip_check(hipEventRecord(e0, s), "event");
-    for (int k = 0; k < reps && r == FF_OK; ++k) r = enqueue_all(b, density, potential, s);
-    if (r == FF_OK) r = hip_check(hipEventRecord(e1, s), "event");
-    if (r == FF_OK) r = hip_check(hipEventSynchronize(e1), "event sync");
-    float ms = 0.f;
-    if (r == FF_OK) r = hip_check(hipEventElapsedTime(&ms, e0, e1), "elapsed");
-    *out = ms / reps;
+    *out = 1e30;
+    for (int round = 0; round < 3; ++round) {  // (the fastest: small batches scatter by half)
+      if (r == FF_OK) r = hip_check(hipEventRecord(e0, s), "event");
+      for (int k = 0; k < reps && r == FF_OK; ++k) r = enqueue_all(b, density, potential, s);
+      if (r == FF_OK) r = hip_check(hipEventRecord(e1, s), "event");
+      if (r == FF_OK) r = hip_check(hipEventSynchronize(e1), "event sync");
+      float ms = 0.f;
+      if (r == FF_OK) r = hip_check(hipEventElapsedTime(&ms, e0, e1), "elapsed");
+      *out = std::min(*out, (double)ms / reps);
+    }
     return r;
   };
   double before = 0.0, after = 0.0;
@@ -681,7 +694,8 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
   int count = 0;
   std::map<std::tuple<int, int, int>, int> seen;  // key -> instance
   for (int i = 0; i < b->count && st == FF_OK; ++i) {
-    const ff_plan* p = b->plans[i];
+    const ff_plan plan = mode_plan(b, i);
+    const ff_plan* p = &plan;
     const int nprec = p->opt.precision == FF_FP64 ? 1 : 2;
     for (int prec = 0; prec < nprec; ++prec) {
       const int M = p->n[2] % 2 ? p->n[2] : p->n[2] / 2;
@@ -692,12 +706,18 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
         // nor have mixed-radix ones
         const MixCfg* mix[4] = {&p->mzr[prec], &p->my[prec], &p->mx[prec], &p->mzi[prec]};
         if (mix[kv[0]]->plan) continue;
-        // z and y passes that run as plane kernels stay so
+        // z and y passes that the batch runs as plane kernels stay so
         if (p->plane[prec] && kv[0] != 2) continue;
         if (!seen.count({kv[0], kv[1], prec})) seen[{kv[0], kv[1], prec}] = i;
       }
     }
   }
+  struct Replaced {
+    int kind, n, prec;
+    bool had;
+    TuneEntry was;
+  };
+  std::vector<Replaced> replaced;  // overrides recorded here, and what was there before
   for (auto& kv : seen) {
     if (st != FF_OK) break;
     const int kind = std::get<0>(kv.first), n = std::get<1>(kv.first), prec = std::get<2>(kv.first);
@@ -759,16 +779,25 @@ ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* 
     }
     if (st == FF_OK && bE) {
       const ff_tune t{kind, n, prec, bE, bT, bF};
-      st = tune_set(&t);
+      Replaced r{kind, n, prec, false, {}};
+      r.had = tune_find(kind, n, prec, r.was);
+      st = tune_set(&t, true);
+      if (st == FF_OK) replaced.push_back(r);
     }
     if (st == FF_OK) count++;
   }
-  if (st == FF_OK) {
+  auto replan = [&]() {
     drop_graph(b);
     b->bound = false;
-    st = make_plans(b);
+    const ff_status r = make_plans(b);
+    return r == FF_OK ? time_batch(&after) : r;
+  };
+  if (st == FF_OK) st = replan();
+  // passes timed alone need not be faster together, beside others: then all go back
+  if (st == FF_OK && after > before && !replaced.empty()) {
+    for (const Replaced& r : replaced) tune_restore(r.kind, r.n, r.prec, r.had ? &r.was : nullptr);
+    st = replan();
   }
-  if (st == FF_OK) st = time_batch(&after);
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   if (st != FF_OK) return st;

@@ -113,8 +113,19 @@ bool row_cfg_with(int nz, int elem_bytes, RowCfg& out, int E, int T, int flags);
 // unchanged where there is no such kernel.
 void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind);
 void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes);
+// Overrides of the register engine's configuration.  One that the batch autotuner
+// recorded (measured) was timed in some plan's register-engine pass: it configures
+// those passes, and takes no other plan off plane kernels or mixed radices, as one set by
+// hand does (tuned_by_hand).
+struct TuneEntry {
+  int E, T, flags;
+  bool measured;
+};
+bool tune_find(int kind, int n, int prec, TuneEntry& out);
 bool tune_lookup(int kind, int n, int prec, int& E, int& T, int& flags);
-ff_status tune_set(const ff_tune* t);
+bool tuned_by_hand(int kind, int n, int prec);
+ff_status tune_set(const ff_tune* t, bool measured = false);
+void tune_restore(int kind, int n, int prec, const TuneEntry* e);  // null: no override
 void tune_reset();
 
 hipError_t launch_col(int E, int f32, int mode, int split, int groups, int blue, int stat, const Launch& l,

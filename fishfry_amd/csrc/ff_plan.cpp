@@ -394,18 +394,38 @@ static std::mutex& tune_mutex() {
   static std::mutex m;
   return m;
 }
-// (kind, n, precision) -> (E, T, flags)
-static std::map<std::tuple<int, int, int>, std::tuple<int, int, int>>& tune_table() {
-  static std::map<std::tuple<int, int, int>, std::tuple<int, int, int>> t;
+// (kind, n, precision) -> override
+static std::map<std::tuple<int, int, int>, TuneEntry>& tune_table() {
+  static std::map<std::tuple<int, int, int>, TuneEntry> t;
   return t;
 }
 
-bool tune_lookup(int kind, int n, int prec, int& E, int& T, int& flags) {
+bool tune_find(int kind, int n, int prec, TuneEntry& out) {
   std::lock_guard<std::mutex> g(tune_mutex());
   auto it = tune_table().find({kind, n, prec});
   if (it == tune_table().end()) return false;
-  std::tie(E, T, flags) = it->second;
+  out = it->second;
   return true;
+}
+
+bool tune_lookup(int kind, int n, int prec, int& E, int& T, int& flags) {
+  TuneEntry e;
+  if (!tune_find(kind, n, prec, e)) return false;
+  E = e.E;
+  T = e.T;
+  flags = e.flags;
+  return true;
+}
+
+bool tuned_by_hand(int kind, int n, int prec) {
+  TuneEntry e;
+  return tune_find(kind, n, prec, e) && !e.measured;
+}
+
+void tune_restore(int kind, int n, int prec, const TuneEntry* e) {
+  std::lock_guard<std::mutex> g(tune_mutex());
+  if (e) tune_table()[{kind, n, prec}] = *e;
+  else tune_table().erase({kind, n, prec});
 }
 
 // Whether the compile-time plan of a kStaticCols entry for (n, E) is the plan
@@ -633,7 +653,7 @@ bool make_row_cfg(int nz, int elem_bytes, RowCfg& out, int kind, int prec) {
   return row_cfg_with(nz, elem_bytes, out, 0, 0, 0);
 }
 
-ff_status tune_set(const ff_tune* t) {
+ff_status tune_set(const ff_tune* t, bool measured) {
   if (!t) return set_error(FF_ERR_INVALID, "ff_tune_set: null");
   if (t->kind < 0 || t->kind > 3 || t->n < 1 || (t->precision != 0 && t->precision != 1))
     return set_error(FF_ERR_INVALID, "ff_tune_set: kind 0..3, n >= 1, precision 0/1");
@@ -656,7 +676,7 @@ ff_status tune_set(const ff_tune* t) {
   }
   if (!ok) return set_error(FF_ERR_INVALID, "ff_tune_set: no valid configuration for that E/T/flags");
   std::lock_guard<std::mutex> g(tune_mutex());
-  tune_table()[{t->kind, t->n, t->precision}] = std::make_tuple(t->E, t->T, t->flags);
+  tune_table()[{t->kind, t->n, t->precision}] = TuneEntry{t->E, t->T, t->flags, measured};
   return FF_OK;
 }
 

@@ -231,8 +231,7 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
   // 131x97x150 FP32 + 2 steps 0.71 and 0.48 ms.
   for (int prec = 0; prec < nprec; ++prec) {
     if (prec && !o.refine_steps) continue;
-    int uE, uT, uF;
-    auto tuned = [&](int kind, int len) { return tune_lookup(kind, len, prec, uE, uT, uF); };
+    auto tuned = [&](int kind, int len) { return tuned_by_hand(kind, len, prec); };
     auto smooth = [](int m) {
       for (int q : {2, 3, 5})
         while (m % q == 0) m /= q;
@@ -242,7 +241,8 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     const long long rows = (long long)n[0] * (n[2] % 2 ? (n[1] + 1) / 2 : n[1]);
     // (odd nz: the pairs of a plane are indexed below 2^16.  Small grids whose odd nz is
     // smooth with few elements per thread stay: 30x25x27, rows 4.4 us and here 6)
-    const bool few = n[2] % 2 && smooth(n[2]) && p->zr[prec].line.E <= 6 && p->N < (1LL << 20);
+    LineCfg line;
+    const bool few = n[2] % 2 && smooth(n[2]) && plan_line(n[2], line) && line.E <= 6 && p->N < (1LL << 20);
     if (!p->fz.n && !few && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
         !(mix_cfg(M, prec, 0, n[1], n[2] % 2, rows, p->mzr[prec]) && mix_cfg(M, prec, 3, n[1], n[2] % 2, rows, p->mzi[prec])))
       p->mzr[prec].plan = p->mzi[prec].plan = nullptr;
@@ -295,15 +295,17 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
   }
 
   // Planes that fit a CU: their z and y passes as one kernel each way, where the
-  // passes would run the same plans in the plain layout.
+  // planner's own passes would run the same plans in the plain layout.
+  auto own_line = [](int len, int E) {
+    LineCfg line;
+    return plan_line(len, line) && line.E == E;
+  };
   for (int prec = 0; prec < nprec; ++prec) {
-    int uE, uT, uF;
     const int kz = plane_index(n[2]), ky = plane_index(n[1]);
     p->planes_fit[prec] =
         kz >= 0 && ky >= 0 && plane_threads(n[2], n[1]) > 0 && !p->pencil && !p->lgKT && !p->slab && !four &&
-        p->zr[prec].line.E == kPlaneLens[kz].ez && p->zi[prec].line.E == kPlaneLens[kz].ez &&
-        p->cy[prec].line.E == kPlaneLens[ky].ey && !tune_lookup(0, n[2] / 2, prec, uE, uT, uF) &&
-        !tune_lookup(3, n[2] / 2, prec, uE, uT, uF) && !tune_lookup(1, n[1], prec, uE, uT, uF);
+        own_line(n[2] / 2, kPlaneLens[kz].ez) && own_line(n[1], kPlaneLens[ky].ey) &&
+        !tuned_by_hand(0, n[2] / 2, prec) && !tuned_by_hand(3, n[2] / 2, prec) && !tuned_by_hand(1, n[1], prec);
   }
   plan_choose_planes(p, 1);
 

@@ -279,8 +279,12 @@ ff_status ff_batch_wait(ff_batch* b, void* stream);
 /* Autotuner: times every valid (elements per thread, lines per workgroup)
  * configuration of each distinct pass of the batch on the given buffers
  * (reps launches each; the buffers' contents are overwritten), records the
- * fastest with ff_tune_set where it beats the plan's own and re-plans.  tuned: passes tuned; ms_before /
- * ms_after: batch solve time before and after. */
+ * fastest as an override where it beats the plan's own kernel and re-plans; where the
+ * batch as a whole is then slower, the overrides go back.  Passes that the batch
+ * runs as plane kernels or in mixed radices are not timed, and no plan
+ * leaves those kernels for an override recorded here (one set with ff_tune_set
+ * keeps a plan on the register engine).  tuned: passes timed; ms_before / ms_after:
+ * batch solve time before and after. */
 ff_status ff_batch_autotune(ff_batch* b, double* const* density, double* const* potential, void* stream, int reps,
                             int* tuned, double* ms_before, double* ms_after);
 ff_status ff_batch_describe(const ff_batch* b, char* buf, size_t len);
