@@ -18,6 +18,8 @@
 
 namespace ff {
 
+struct LineCfg;
+
 constexpr int kMixStages = 10;
 constexpr int kMixThreads = 256;
 
@@ -72,9 +74,10 @@ std::vector<int> mix_radices(int n);
 // The plan and tile of a pass of kind 1 (y columns), 2 (x columns), 0 (z forward
 // rows) or 3 (z inverse rows) over lines of n, with its tables resident on the
 // current device; ncols: the lines of a plane (columns); pairs: rows of odd nz,
-// two to a line; lines: all the lines of the pass.  False where the
-// length has no plan, no tile fits the LDS, or a table could not be allocated.
-bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, long long lines, MixCfg& out);
+// two to a line; lines: all the lines of the pass; engine: the register engine's
+// line.  False where the length has no plan, no tile fits the LDS, the engine is the
+// faster one, or a table could not be allocated.
+bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, long long lines, const LineCfg& engine, MixCfg& out);
 
 hipError_t mix_col(int f32, int mode, const Launch& l, const ColArgs& a);
 hipError_t mix_r2c(int f32, int in_f32, int odd, const Launch& l, const RowArgs& a);

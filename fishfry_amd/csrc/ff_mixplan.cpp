@@ -110,7 +110,34 @@ static void build_plan(int n, int prec, std::vector<unsigned char>& buf) {
   memcpy(buf.data(), &mp, sizeof mp);
 }
 
-bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, long long lines, MixCfg& out) {
+// Whether Bluestein's transforms in the register engine (line e) are the faster ones
+// for a pass of so many tiles.  A tile's own time counts where the tiles do not fill
+// the chip: eight lines by 256 threads take n * (radices) steps, the engine's up
+// to 512 threads and more the same few passes for every n up to the next engine length.
+// Measured (MI355X; engine and mixed radices; about 150 tiles, and 1000 or more):
+//   FP32 + 1 step 969x20x60  271 and 387 us, 566 213 and 270, 493 177 and 221, 731 303 and 304;
+//     at 64x256 columns 493 and 566 are 0.6-0.9 of the engine, 969 1.15 of it
+//   FP64 y passes 398  15.3 and 20.7 us, 501 16.1 and 24.9 (large: 0.3-1.1 of the engine),
+//     969 200 and 251 us at 64x256
+//   FP64 odd rows 283 of 768 rows  12.8 and 18.6 us, of 12288 0.4 of the engine.
+static bool engine_faster(int n, int prec, int kind, bool pairs, long long tiles, const std::vector<int>& rs,
+                          const LineCfg& e) {
+  const int D = rs.back();
+  if (D <= 13) return false;
+  const bool few = tiles < 256, rows = kind == 0 || kind == 3;
+  const bool two = rs.size() > 1 && rs[rs.size() - 2] > 13;  // dense stages
+  if (two && n >= 965 && !rows) return true;
+  if (!few) return false;
+  if (two && n >= 480 && prec) return !pairs || e.lp.n <= 1296;
+  if (pairs) return !prec && D > 200;
+  if (prec) {
+    const double cost = (double)e.lp.n * (e.lp.np + 0.04 * e.E) / n;  // (as plan_line's)
+    return (n > 864 && !rows) || (D > 200 && n >= 2 * D && cost < 8.7);
+  }
+  return kind == 1 && D >= 130 && n >= 2 * D && e.E <= 16 && e.lp.n <= 1024;
+}
+
+bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, long long lines, const LineCfg& engine, MixCfg& out) {
   out = MixCfg{};
   const std::vector<int> rs = mix_radices(n);
   const bool rows = kind == 0 || kind == 3;
@@ -138,6 +165,7 @@ bool mix_cfg(int n, int prec, int kind, int ncols, bool pairs, long long lines, 
   while (T > 1 && bytes(T) > 160 * 1024) T /= 2;
   while (!rows && T > 1 && T / 2 >= ncols) T /= 2;
   if (bytes(T) > 160 * 1024) return false;
+  if (engine_faster(n, prec, kind, pairs, (lines + T - 1) / T, rs, engine)) return false;
   // (the index divisions are exact below 2^16)
   if ((long long)T * (n + 2) >= 65536) return false;
   out.T = T;

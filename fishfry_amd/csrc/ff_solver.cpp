@@ -239,19 +239,30 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     };
     const int M = n[2] % 2 ? n[2] : n[2] / 2;
     const long long rows = (long long)n[0] * (n[2] % 2 ? (n[1] + 1) / 2 : n[1]);
-    // (odd nz: the pairs of a plane are indexed below 2^16.  Small grids whose odd nz is
-    // smooth with few elements per thread stay: 30x25x27, rows 4.4 us and here 6)
+    // (odd nz: the pairs of a plane are indexed below 2^16.)  Odd smooth rows that the
+    // register engine transforms in few passes stay there: 3^k and 5^k (E to 6) but for
+    // 243 and 729 of large FP64 solves, and FP32 rows of large grids that take four passes
+    // or fewer.  Engine and pairs, us: FP64 z forward 128x128x125 9.2 and 10.7,
+    // 320x320x125 36 and 55, x625 253 and 294, x243 155 and 119, 96x97x243 14.4 and
+    // 15.8; FP32 + 1 step 128x128x125 154 and 211, 128x128x729 with pairs in its residual
+    // only 567 and 595; FP32 passes alone at 225 and 375 0.9 of the engine to 10^6 points and
+    // 1.02-1.12 of it beyond, 675 0.9.
     LineCfg line;
-    const bool few = n[2] % 2 && smooth(n[2]) && plan_line(n[2], line) && line.E <= 6 && p->N < (1LL << 20);
-    if (!p->fz.n && !few && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
-        !(mix_cfg(M, prec, 0, n[1], n[2] % 2, rows, p->mzr[prec]) && mix_cfg(M, prec, 3, n[1], n[2] % 2, rows, p->mzi[prec])))
+    bool engine = false;
+    if (n[2] % 2 && smooth(n[2]) && plan_line(n[2], line)) {
+      if (line.E <= 6) engine = o.precision != FF_FP64 || line.lp.np < 5 || p->N < (5LL << 19);
+      else engine = prec && line.lp.np < 5 && p->N >= (1LL << 20);
+    }
+    if (!p->fz.n && !engine && (n[2] % 2 ? n[1] < 65536 : !smooth(M)) && !tuned(0, M) && !tuned(3, M) &&
+        !(mix_cfg(M, prec, 0, n[1], n[2] % 2, rows, p->zr[prec].line, p->mzr[prec]) &&
+          mix_cfg(M, prec, 3, n[1], n[2] % 2, rows, p->zi[prec].line, p->mzi[prec])))
       p->mzr[prec].plan = p->mzi[prec].plan = nullptr;
     const bool pen = p->pencil && prec == mainp;
     const long long yl = (long long)n[0] * p->nh, xl = (long long)n[1] * p->nh;
     if (!p->fy.n && !smooth(n[1]) && !tuned(1, n[1]))
-      mix_cfg(n[1], prec, 1, pen ? std::max(p->nh, n[0]) : p->nh, false, yl, p->my[prec]);
+      mix_cfg(n[1], prec, 1, pen ? std::max(p->nh, n[0]) : p->nh, false, yl, p->cy[prec].line, p->my[prec]);
     if (!p->fx.n && !p->fy.n && !smooth(n[0]) && !tuned(2, n[0]))
-      mix_cfg(n[0], prec, 2, pen ? n[1] : p->nh, false, xl, p->mx[prec]);
+      mix_cfg(n[0], prec, 2, pen ? n[1] : p->nh, false, xl, p->cx[prec].line, p->mx[prec]);
     // one workgroup per tile of a 32-bit grid
     auto fits = [&](MixCfg& c, long long planes, long long lines) {
       if (c.plan && planes * ((lines + c.T - 1) / c.T) > INT_MAX) c.plan = nullptr;

@@ -4,11 +4,13 @@ test_gpu_mixed.py compare, so that those comparisons are with another kernel; no
 them under the overrides that those tests use, nor where a rule excludes them."""
 import json
 
+import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
 
 import fishfry_amd as ff  # noqa: E402
+import oracle  # noqa: E402
 from test_gpu_mixed import LENGTHS  # noqa: E402
 from test_gpu_plane import SHAPES  # noqa: E402
 
@@ -53,7 +55,8 @@ def largest_prime(n):
 @pytest.mark.parametrize("n", LENGTHS)
 def test_mixed(n):
     top = largest_prime(n)
-    for prec, key, limit, pairs in ((0, "mixed", 200, 300), (1, "mixed_fp32", 300, 420)):
+    # (pairs of FP64 rows to 300 only where their tiles fill the chip: test_engine_by_size)
+    for prec, key, limit, pairs in ((0, "mixed", 200, 200), (1, "mixed_fp32", 300, 420)):
         kw = REFINED if prec else {}
         for g, axes, most in (((n, 6, 10), ["x"], limit), ((5, n, 8), ["y"], limit), ((3, 4, 2 * n), ["z", "zi"], limit),
                               ((4, 5, n), ["z", "zi"], pairs)):
@@ -69,6 +72,38 @@ def test_mixed(n):
             assert "y" not in described((5, n, 8), **kw)[key]
         finally:
             ff.tune_reset()
+
+
+# length, axis and grid: mixed radices in FP64 and in refined FP32, or the register engine
+SIZES = [
+    # odd rows of 2^a 3^b 5^c: 3^k and 5^k, and 3^a 5^b of few and many engine passes
+    ("z", (128, 128, 125), (0, 0)), ("z", (8, 8, 125), (0, 0)), ("z", (96, 97, 243), (0, 0)),
+    ("z", (128, 128, 243), (1, 0)), ("z", (31, 45, 225), (1, 1)), ("z", (96, 97, 225), (1, 0)),
+    ("z", (96, 97, 675), (1, 1)), ("z", (31, 45, 729), (0, 0)), ("z", (64, 64, 729), (1, 0)),
+    # dense stages where the tiles do not fill the chip, and where they do
+    ("z", (16, 48, 283), (0, 1)), ("z", (64, 66, 283), (1, 1)), ("x", (969, 20, 60), (0, 0)),
+    ("y", (96, 969, 62), (0, 0)), ("y", (20, 566, 60), (0, 0)), ("y", (96, 566, 62), (0, 1)),
+    ("y", (20, 493, 60), (1, 0)), ("y", (96, 493, 62), (1, 1)), ("y", (20, 398, 60), (0, 1)),
+    ("y", (96, 398, 62), (1, 1)), ("x", (940, 20, 60), (1, 0)), ("x", (940, 96, 62), (1, 1)),
+]
+
+
+@pytest.mark.parametrize("axis,n,want", SIZES)
+def test_engine_by_size(axis, n, want):
+    got = (described(n)["mixed"], described(n, precision=ff.FF_FP32_REFINE, refine_steps=1)["mixed_fp32"])
+    assert tuple(int(axis in g) for g in got) == want
+    f = np.random.default_rng(sum(n)).standard_normal(n)
+    w = oracle.solve(f)
+    lo, hi, _ = ff.benchmark_grid(n)
+    for kw in (dict(), REFINED):
+        with ff.ParisPencil(n, lo, hi, **kw) as p:
+            d = torch.zeros(p.bytes() // 8, dtype=torch.float64, device="cuda")
+            phi = torch.full_like(d, float("nan"))
+            d[:f.size] = torch.from_numpy(f.reshape(-1)).cuda()
+            print("size", n, kw, flush=True)
+            p.solve(p.bytes(), d, phi)
+            e = np.linalg.norm(phi[:f.size].cpu().numpy().reshape(n) - w) / np.linalg.norm(w)
+            assert e < (1e-13 if not kw else 1e-12), e  # as in test_gpu_mixed.py
 
 
 def test_groups_and_long_descriptions():
