@@ -112,7 +112,7 @@ bool row_cfg_with(int nz, int elem_bytes, RowCfg& out, int E, int T, int flags);
 // a default one (the same elements per thread, hence the same results to the bit);
 // unchanged where there is no such kernel.
 void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind);
-void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes);
+void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes, int kind, long long rows);
 // Overrides of the register engine's configuration.  One that the batch autotuner
 // recorded (measured) was timed in some plan's register-engine pass: it configures
 // those passes, and takes no other plan off plane kernels or mixed radices, as one set by

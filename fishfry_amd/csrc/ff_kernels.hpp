@@ -974,9 +974,14 @@ constexpr int kNumStaticRows = sizeof(kStaticRows) / sizeof(kStaticRows[0]);
 //   240^3    97   83  138   83   83     70   50   76   48   59
 //   1000^3 3088 4426 5184 3915 3426   2908 3579 4553 3232 3291  (of them x compiled in before)
 // What bounds them now is memory: 2.4-2.5 ms is 4.8 TB/s at 900^3.
+// few (rows): the FP64 z inverse takes the kernel to kLdsFewRows rows only and the generic
+// one beyond, where its memory twiddles are no bound and LDS is (generic and this: 800 rows of
+// 320 9.5 and 9.1 us, 30720 41 and 49, 160000 184 and 230; 512x512x640 718 and 793;
+// 800^3 2250 and 2620; 30720 rows of 144 16.5 and 20.0).
 struct LdsLine {
-  int n, E;
+  int n, E, few;
 };
+constexpr long long kLdsFewRows = 8192;
 constexpr LdsLine kLdsCols[] = {{36, 6}, {40, 20}, {45, 15}, {50, 10}, {54, 6}, {60, 30},
     {72, 12}, {75, 15}, {80, 20}, {81, 3}, {90, 30}, {100, 10}, {108, 6}, {120, 30}, {125, 5},
     {135, 15}, {144, 12}, {150, 30}, {160, 20}, {162, 6}, {180, 30}, {192, 12}, {200, 10}, {216, 6},
@@ -986,10 +991,10 @@ constexpr LdsLine kLdsCols[] = {{36, 6}, {40, 20}, {45, 15}, {50, 10}, {54, 6}, 
     {750, 30}, {768, 12}, {768, 24}, {800, 20}, {810, 30}, {864, 12}, {900, 30}, {960, 30}, {972, 6}, {1000, 10},
     {1000, 20}};
 constexpr LdsLine kLdsRows[] = {{18, 6}, {20, 10}, {25, 5}, {27, 3}, {30, 30}, {36, 6}, {40, 20}, {45, 15},
-    {50, 10}, {54, 6}, {60, 30}, {72, 12}, {75, 15}, {81, 3}, {90, 30}, {96, 24}, {100, 10}, {108, 6}, {120, 30},
-    {125, 5}, {135, 15}, {144, 12}, {150, 30}, {160, 20}, {162, 6}, {180, 30}, {192, 12}, {200, 10}, {216, 6},
-    {225, 15}, {240, 30}, {243, 3}, {250, 10}, {270, 30}, {288, 12}, {300, 30}, {320, 20}, {324, 6}, {360, 30},
-    {375, 15}, {400, 20}, {405, 15}, {432, 12}, {450, 30}, {480, 30}, {486, 6}};
+    {50, 10}, {54, 6}, {60, 30}, {72, 12, 1}, {75, 15}, {81, 3}, {90, 30}, {96, 24}, {100, 10}, {108, 6}, {120, 30},
+    {125, 5}, {135, 15}, {144, 12}, {150, 30}, {160, 20, 1}, {162, 6}, {180, 30}, {192, 12}, {200, 10}, {216, 6},
+    {225, 15}, {240, 30}, {243, 3}, {250, 10}, {270, 30}, {288, 12}, {300, 30}, {320, 20, 1}, {324, 6}, {360, 30},
+    {375, 15}, {400, 20, 1}, {405, 15}, {432, 12}, {450, 30}, {480, 30}, {486, 6}};
 constexpr int kNumLdsCols = sizeof(kLdsCols) / sizeof(kLdsCols[0]);
 constexpr int kNumLdsRows = sizeof(kLdsRows) / sizeof(kLdsRows[0]);
 // stat of these kernels, and the kernels of a line (null: none); ff_lines.hip

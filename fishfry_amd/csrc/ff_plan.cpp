@@ -528,13 +528,19 @@ void col_lds_twiddles(ColCfg& c, int ncols, int elem_bytes, int kind) {
   c.threads = s.threads;
 }
 
-void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes) {
+void row_lds_twiddles(RowCfg& c, int nz, int elem_bytes, int kind, long long rows) {
   if (nz % 2 || c.line.bluestein() || c.stat == 2) return;
   const int M = nz / 2;
   // (compiled-in rows within a wavefront, which exchange without a workgroup barrier, gain
   // nothing from it: 128^3 FP64 50.5 us with twiddles from memory, 53.4 from LDS)
   if (c.stat && 64 % (M / c.line.E) == 0) return;
+  // (rows of 500: 800 rows 6.9 us from memory and 7.6 from LDS, 3000 12.6 and 14.5, 30720
+  // 105 and 100)
+  if (c.stat && rows <= kLdsFewRows) return;
   if (!c.stat && !lds_line_matches<kLdsRows, kNumLdsRows>(M, c.line.E, c.line.lp)) return;
+  if (kind == 3 && elem_bytes == 16 && rows > kLdsFewRows)
+    for (const LdsLine& l : kLdsRows)
+      if (l.few && l.n == M && l.E == c.line.E) return;
   const size_t lds = c.lds + (size_t)tw_lds_slots(M) * elem_bytes;
   if (lds > 160 * 1024) return;
   c.lds = lds;

@@ -297,8 +297,9 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
     int uE, uT, uF;
     const int eb = prec ? 8 : 16;
     const bool pen = p->pencil && prec == mainp;
-    if (!p->fz.n && !tune_lookup(0, n[2] / 2, prec, uE, uT, uF)) row_lds_twiddles(p->zr[prec], n[2], eb);
-    if (!p->fz.n && !tune_lookup(3, n[2] / 2, prec, uE, uT, uF)) row_lds_twiddles(p->zi[prec], n[2], eb);
+    const long long rows = (long long)n[0] * n[1];
+    if (!p->fz.n && !tune_lookup(0, n[2] / 2, prec, uE, uT, uF)) row_lds_twiddles(p->zr[prec], n[2], eb, 0, rows);
+    if (!p->fz.n && !tune_lookup(3, n[2] / 2, prec, uE, uT, uF)) row_lds_twiddles(p->zi[prec], n[2], eb, 3, rows);
     if (!p->fy.n && !tune_lookup(1, n[1], prec, uE, uT, uF))
       col_lds_twiddles(p->cy[prec], pen ? std::min(p->nh, n[0]) : p->nh, eb, 1);
     if (!p->fx.n && !p->fy.n && !tune_lookup(2, n[0], prec, uE, uT, uF))

@@ -106,6 +106,42 @@ def test_engine_by_size(axis, n, want):
             assert e < (1e-13 if not kw else 1e-12), e  # as in test_gpu_mixed.py
 
 
+@pytest.mark.parametrize("m", [72, 160, 320, 400, 500])
+def test_row_lines_by_size(m):
+    """Rows whose kernel depends on their number: the FP64 z inverse of some lengths is the generic
+    one beyond 8192 rows, rows of 500 take their twiddles from LDS beyond them; one result."""
+    def lds(n):
+        d = described(n)
+        try:
+            for kind in (0, 3):
+                t = ff.tune_query(kind, m, 0, m + 1)
+                ff.tune_set(kind, m, 0, t.E, t.T, ff.FF_TUNE_GENERIC)
+            g = described(n)
+        finally:
+            ff.tune_reset()
+        return d["z"]["lds"] > g["z"]["lds"], d["zi"]["lds"] > g["zi"]["lds"]
+
+    few, many = (64, 128, 2 * m), (64, 129, 2 * m)
+    assert lds(few) == ((False, False) if m == 500 else (True, True))
+    assert lds(many) == ((True, True) if m == 500 else (True, False))
+    f = torch.from_numpy(np.random.default_rng(m).standard_normal(many)).cuda()
+    lo, hi, _ = ff.benchmark_grid(many)
+    out = []
+    for tuned in (0, 1):
+        try:
+            for kind in (0, 3) if tuned else ():
+                t = ff.tune_query(kind, m, 0, m + 1)
+                ff.tune_set(kind, m, 0, t.E, t.T, ff.FF_TUNE_GENERIC)
+            with ff.ParisPencil(many, lo, hi) as p:
+                d = torch.zeros(p.bytes() // 8, dtype=torch.float64, device="cuda")
+                d[:f.numel()] = f.reshape(-1)
+                out.append(torch.full_like(d, float("nan")))
+                p.solve(p.bytes(), d, out[-1])
+        finally:
+            ff.tune_reset()
+    assert torch.equal(out[0][:f.numel()], out[1][:f.numel()])
+
+
 def test_groups_and_long_descriptions():
     """Planes that a group fills the chip with, and a batch whose plans' descriptions are long."""
     b = ff.Batch([dict(n=(40, 128, 128))] * 5, flags=ff.FF_BATCH_GROUPED)
