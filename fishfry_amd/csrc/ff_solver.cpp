@@ -352,7 +352,8 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
 
   // twiddle tables of the engine transforms (length m for Bluestein lines),
   // the even-nz post-twiddles and the Bluestein tables, from the resident
-  // per-device cache (shared by every plan with the same line lengths)
+  // per-device cache (shared by every plan with the same line lengths); a pass in
+  // mixed radices has its own and takes none of the engine's
   const int nz = n[2];
   bool ok = true;
   auto blue = [&](const LineCfg& c, int prec, const void* (&o)[3]) {
@@ -362,7 +363,7 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
   for (int prec = 0; prec < nprec && ok; ++prec) {
     p->tw_zpost[prec] = table_post(nz, prec);
     ok = p->tw_zpost[prec] != nullptr;
-    if (!p->fz.n) {
+    if (!p->fz.n && !(p->mzr[prec].plan && p->mzi[prec].plan)) {
       p->tw_z[prec] = table_twiddle(p->zr[prec].line.lp.n, prec);
       p->tw_zi[prec] = table_twiddle(p->zi[prec].line.lp.n, prec);
       ok = ok && p->tw_z[prec] && p->tw_zi[prec];
@@ -382,7 +383,7 @@ ff_status plan_create(const int n[3], const double lo[3], const double hi[3], co
         ok = ok && fs.tw1[prec] && fs.tw2[prec] && fs.twn[prec];
         blue(fs.c1[prec].line, prec, fs.bl1[prec]);
         blue(fs.c2[prec].line, prec, fs.bl2[prec]);
-      } else {
+      } else if (!(axis ? p->my : p->mx)[prec].plan) {
         const void*& tw = axis ? p->tw_y[prec] : p->tw_x[prec];
         tw = table_twiddle(c.line.lp.n, prec);
         ok = ok && tw;
