@@ -125,7 +125,6 @@ struct ColArgs {
   // spectral filter); the axis term is g[k] * dd
   const double *symx, *symy, *symz;
   double* dc_out;  // FILTER / SYMBOL: receives the forward (0,0,0) term (sum of the input)
-  int dc_add;      // it is added to what dc_out holds (FP32 passes: the sum a correction's residual still has)
   const void* tw;
   LinePlan lp;
   int nline;                     // transform length (lp.n: engine length; larger for Bluestein)
@@ -133,6 +132,7 @@ struct ColArgs {
   const PassInst* inst;           // grouped launch: per-instance fields (null: one solve)
   const void* mix;                // the MixPlan of a mixed-radix pass, in device memory (null: none)
   int nbuf;                       // its LDS buffers
+  int dc_add;                     // dc_out is added to (FP32 passes: the sum a correction's residual still has)
 };
 
 // Buffers in global memory.  The per-instance fields come either from the
