@@ -938,8 +938,8 @@ struct StaticCol {
                   // many waves per SIMD
 };
 constexpr StaticCol kStaticCols[] = {{1024, 16, 4, 0, 0, 2, 6, 2}, {1024, 16, 8, 1, 0, 2, 6, 2}, {1024, 16, 4, 0, 1, 3, 6, 3},
-                                     // x passes only at 512, 768 and 1000 (the y passes are as fast or
-                                     // faster generic there); both column passes at 256 and below
+                                     // x passes only at 512, 768 and 1000 (the y passes take the lines
+                                     // of kLdsCols); both column passes at 256 and below
                                      {768, 12, 4, 0, 0, 3, 4}, {1000, 20, 4, 0, 0, 2, 4},
                                      {512, 8, 4, 0, 0, 4, 4}, {256, 16, 16, 0, 0, 2, 6}, {128, 16, 32, 0, 0, 2, 6},
                                      // small grids (FP64 and FP32)

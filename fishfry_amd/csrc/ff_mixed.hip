@@ -7,10 +7,11 @@
 // their four transforms of at least twice the length and by the registers of
 // the kernels that hold them (x 1.27 ms, y 0.32, z forward 0.50, z inverse 0.61);
 // here x takes 0.31 ms, y 0.22, z 0.18 and 0.20, bound by the LDS exchanges and
-// index arithmetic of the stages.  A tile is about 2048 FP64 (4096 FP32) values,
-// 32 to 50 KB of LDS in two buffers, so three or four workgroups of 256 threads
-// share a CU and one's memory phase covers another's stages; columns keep
-// row segments of 64 bytes and more.  Two buffers in turn cost one barrier per
+// index arithmetic of the stages.  A tile is about 2048 FP64 (4096 FP32) values
+// in two buffers (49 KB of LDS at 385), more where row segments of 64 bytes and the
+// eight lines of a dense stage ask for it (67 KB at 127, 132 KB at 1017 in FP64), so that two
+// to four workgroups of 256 threads share a CU, one at the longest lines, and one's memory
+// phase covers another's stages.  Two buffers in turn cost one barrier per
 // stage instead of two, and let a stage's butterflies be spread over all
 // threads whatever its radix.
 #include <type_traits>

@@ -13,7 +13,10 @@ namespace ff {
 // planner's defaults), so the results are theirs bit for bit.  The plan is used
 // where the planner's agrees.  Rows of 160 and more would leave a plane of
 // complex values no room in LDS; exchanging real and imaginary parts one after
-// the other instead doubles the barriers, and was slower than the passes.
+// the other instead doubles the barriers, and was slower than the passes.  (These are
+// the lengths that were measured, the batches' and other round ones; 54, 60, 75, 81, 90,
+// 120 and 125 would fit and are not compiled in: every row length takes a kernel for each
+// column length.)
 struct PlaneLen {
   int n, ez, ey;  // nz or ny; elements per thread of the row (0: columns only) and of the column
 };

@@ -38,7 +38,7 @@ struct StencilArgs {
   const double* f;
   void* out;           // float r (residual) or double L_h phi
   int nx, ny, nz;
-  int lgtk;            // log2 of TK (z positions per tile); TJ = 256 / TK rows
+  int lgtk;            // log2 of TK (z positions per tile); TJ = kStencilThreads / TK rows
   int tiles_j, tiles_k, chunks, chunk;  // workgroup grid: tiles_j * tiles_k * chunks; planes per chunk
   double cx, cy, cz;   // 1/h^2 per axis (5-point: divided by 12)
   double scale;        // 1/(nx ny nz)
